@@ -75,7 +75,7 @@ struct als_engine {
     float *t_val = nullptr;
     float *U = nullptr, *V = nullptr;  // FP32 factors, row stride ld
     uint16_t *Us = nullptr, *Vs = nullptr;  // 16-bit shadows (mixed precision)
-    int *queue = nullptr;              // 4 ints: update kernel's queue pair, dual kernel's
+    int *queue = nullptr;              // ticket counters: update kernel's ([0]), dual kernel's ([2])
     int *fail = nullptr;               // 1 int
     double *partials = nullptr, *dsum = nullptr;
     int rmse_blocks = RMSE_BLOCKS;
@@ -314,14 +314,16 @@ int launch_schedule(als_engine *e, const Side &s, const float *Y, const uint16_t
     if (solve == SOLVE_CHOL) a.refine = 0;
     // the side's kernel variant applies to the engine's own solver
     const int var = solve == e->solve ? s.variant : 0;
-    const int ugrid = var ? e->grid_v1 : s.grid;
+    // no more waves than batches: a wave without one only costs its launch
+    const int umax = var ? e->grid_v1 : s.grid;
+    const int ugrid = std::min(umax, s.nbatches), dgrid = std::min(e->dual_grid, s.dnbatches);
     if (beside && e->dual_beside && !Lsave && s.nbatches > 0 && s.dnbatches > 0) {
         UpdateArgs d = dual_args(s, a);
         d.queue = e->queue + 2;
         HIPCHK(e, hipEventRecord(e->dual_fork, st));
         HIPCHK(e, hipStreamWaitEvent(e->dual_stream, e->dual_fork, 0));
         HIPCHK(e, launch_update(e->T, e->prec, solve, var, a, ugrid, e->lds, st));
-        HIPCHK(e, launch_dual(e->T, e->prec, solve, d, e->dual_grid, e->dual_lds, e->dual_stream));
+        HIPCHK(e, launch_dual(e->T, e->prec, solve, d, dgrid, e->dual_lds, e->dual_stream));
         HIPCHK(e, hipEventRecord(e->dual_join, e->dual_stream));
         HIPCHK(e, hipStreamWaitEvent(st, e->dual_join, 0));
         return ALS_OK;
@@ -329,8 +331,8 @@ int launch_schedule(als_engine *e, const Side &s, const float *Y, const uint16_t
     if (s.nbatches > 0) HIPCHK(e, launch_update(e->T, e->prec, solve, var, a, ugrid, e->lds, st));
     if (s.dnbatches > 0) {
         const UpdateArgs d = dual_args(s, a);
-        if (Lsave) HIPCHK(e, launch_update(e->T, e->prec, solve, var, d, ugrid, e->lds, st));
-        else HIPCHK(e, launch_dual(e->T, e->prec, solve, d, e->dual_grid, e->dual_lds, st));
+        if (Lsave) HIPCHK(e, launch_update(e->T, e->prec, solve, var, d, std::min(umax, s.dnbatches), e->lds, st));
+        else HIPCHK(e, launch_dual(e->T, e->prec, solve, d, dgrid, e->dual_lds, st));
     }
     return ALS_OK;
 }

@@ -29,7 +29,7 @@ struct UpdateArgs {
     float *partial;             // partial Gram tiles, NT*256 floats per slot
     const int *batch_begin;     // batch b = units[batch_begin[b] .. batch_begin[b+1])
     int nbatches;
-    int *queue;                 // [0] next batch, [1] waves that left
+    int *queue;                 // next ticket (0 between launches)
     int cg_iters;
     float cg_tol;
     int cg_fp16_a;              // CG on an FP16-rounded A

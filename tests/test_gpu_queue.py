@@ -1,0 +1,57 @@
+"""The update kernels' work queue where the batches just fill the launched
+waves: as many batches as waves, one more, one fewer, a single wave and a
+single batch. Each half-sweep runs several times on one engine (the ticket
+counter has to be back at zero after every launch), directly and as replays
+of a captured sweep, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+import cuda_als_amd as ca
+from cuda_als_amd import engine as E
+from oracle import als_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+ROWS, COLS, PER_ROW = 96, 40, 9
+
+
+def matrix():
+    """Every user has PER_ROW ratings, so a batch of work 1 is one row."""
+    rng = np.random.default_rng(5)
+    idx = np.concatenate([np.sort(rng.choice(COLS, PER_ROW, replace=False)) for _ in range(ROWS)])
+    val = rng.integers(1, 6, idx.size)
+    return ca.from_arrays(ROWS, COLS, np.arange(ROWS + 1) * PER_ROW, idx, val, [0], [0], [3.0])
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("grid", [1, 2, ROWS - 1, ROWS, ROWS + 1])
+@pytest.mark.parametrize("f,prec", [(16, E.Prec.FP32), (70, E.Prec.FP16)])
+def test_batches_against_waves(f, prec, grid, graph):
+    """f = 70 sends every row here through the dual kernel unless its limit is
+    0; both are run. FP32 factors within 1e-4 of the oracle on the exact
+    factors (as elsewhere for one half-sweep), FP16 within 1e-4 on the
+    rounded ones."""
+    d = matrix()
+    V0 = np.random.default_rng(1).standard_normal((COLS, f)).astype(np.float32) * 0.3
+    want = O.update_rows(O.config(f, 0.05, O.SOLVE_CHOL, gram_prec=O.PREC_FP16 if prec == E.Prec.FP16 else O.PREC_EXACT),
+                         np.arange(ROWS), d.csr_ptr, d.csr_idx, d.csr_val, V0.astype(np.float64))
+    with E.Engine(E.make_config(f, 0.05, 1, E.SolveType.CHOL, prec, use_graph=graph, batch_work=1), d) as e:
+        for limit in {0, e.info().dual_max}:
+            e.set_grid(ca.ALS_SIDE_USERS, grid)
+            e.set_dual_limit(ca.ALS_SIDE_USERS, limit)
+            first = None
+            for _ in range(4):
+                e.set_factors(ca.ALS_SIDE_USERS, np.zeros((ROWS, f), np.float32))
+                e.set_factors(ca.ALS_SIDE_ITEMS, V0)
+                (e.sweep if graph else lambda: e.update(ca.ALS_SIDE_USERS))()
+                U = e.get_factors(ca.ALS_SIDE_USERS)
+                first = U if first is None else first
+                assert np.array_equal(U, first)
+            err = np.abs(first - want).max(axis=1) / np.maximum(1.0, np.abs(want).max(axis=1))
+            assert e.info().failures == 0 and err.max() <= 1e-4, err.max()
+            # one batch for all rows
+            e.set_schedule(ca.ALS_SIDE_USERS, 0, 1 << 30)
+            e.set_factors(ca.ALS_SIDE_ITEMS, V0)
+            e.update(ca.ALS_SIDE_USERS)
+            assert np.array_equal(e.get_factors(ca.ALS_SIDE_USERS), first)
+            e.set_schedule(ca.ALS_SIDE_USERS, 0, 1)
