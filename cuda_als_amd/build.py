@@ -56,10 +56,11 @@ def build_lib() -> Path:
     OBJ.mkdir(exist_ok=True)
     jobs: list[list[str]] = []
     objs: list[Path] = []
-    for p in (0, 1, 2):
-        for unit in ("als_update",):
-            o = OBJ / f"{unit}_p{p}.o"
-            jobs.append([HIPCC, *HIP_FLAGS, f"-DALS_PREC={p}", "-c", str(CSRC / f"{unit}.hip"), "-o", str(o)])
+    for aug in (1, 0):
+        for p in (0, 1, 2):
+            o = OBJ / f"als_update_p{p}{'ba'[aug]}.o"
+            jobs.append([HIPCC, *HIP_FLAGS, f"-DALS_PREC={p}", f"-DALS_AUG={aug}", "-c",
+                         str(CSRC / "als_update.hip"), "-o", str(o)])
             objs.append(o)
     # every other HIP unit of csrc/, plus the host units that call the HIP runtime
     hip_units = sorted(p.name for p in CSRC.glob("*.hip") if p.name != "als_update.hip")

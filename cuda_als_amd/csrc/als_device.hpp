@@ -107,9 +107,14 @@ template <> __device__ __forceinline__ float from16<PREC_FP16>(uint16_t h) {
 #define ALS_DUAL_TD_MAX 5
 #endif
 
-template <int T, int E> struct Geo {
+template <int T, int E, bool AUG = true> struct Geo {
     static constexpr int NT = T * (T + 1) / 2;  // lower-triangle 16x16 tiles
-    static constexpr int FP = 16 * T;           // padded augmented dimension
+    static constexpr int FP = 16 * T;           // padded dimension of the system
+    // Row stride of the factor matrices: always that of the augmented system
+    static constexpr int LD = AUG ? FP : FP + 16;
+    // Floats of one part of a split row: the tiles and, where it is not in
+    // them, b
+    static constexpr int PART = NT * 256 + (AUG ? 0 : FP);
     static constexpr int YT_H = 40;             // 16-bit stage row: 32 ratings + 8 pad (80 B)
     // Factor row j of the 16-bit stage sits at row j + j / 8: the gather
     // writes rows 8s + 2v (s = 0..12 in one instruction) and the MFMA reads
@@ -124,13 +129,15 @@ template <int T, int E> struct Geo {
     // 2 * RS16 bytes an odd multiple of 32 modulo 256, or T = 2 mod 4, the
     // four land on distinct LDS banks.
     static constexpr int RS16 = (T % 4 == 0) ? FP + 16 : FP;
-    // Rows with fewer than 16 * DUAL_TD ratings take the dual system (T >= 5).
-    static constexpr int DUAL_TD = T >= 5 ? (T - 2 < ALS_DUAL_TD_MAX ? T - 2 : ALS_DUAL_TD_MAX) : 0;
+    // Rows with fewer than 16 * DUAL_TD ratings take the dual system (f >= 64).
+    static constexpr int TA = AUG ? T : T + 1;  // blocks of the augmented system
+    static constexpr int DUAL_TD = TA >= 5 ? (TA - 2 < ALS_DUAL_TD_MAX ? TA - 2 : ALS_DUAL_TD_MAX) : 0;
     // The double-buffered LDS-DMA Gram (gram_row16_dma): two rating-major
     // buffers of CHUNK x FP halves, then a second ibuf/rbuf pair (256 bytes).
-    // Used where a row of FP halves keeps a transposing read's four rows on
-    // distinct LDS banks (T % 4 != 0) and a chunk's tasks fit a wave (T <= 8).
-    static constexpr bool DMA_GRAM = gram_dma_built(T, E);
+    // A chunk's tasks must fit a wave (T <= 8). Where T % 4 == 0 the stage's
+    // 32-byte column blocks are permuted by row (gram_dma_loop) to keep a
+    // transposing read's four rows on distinct LDS banks.
+    static constexpr bool DMA_GRAM = gram_dma_built(TA, E);
     static constexpr int DMA_STAGE_BYTES = 2 * CHUNK * FP * 2 + 256;
     static constexpr int GRAM_STAGE_BYTES =
         E == PREC_FP32 ? CHUNK * YR * 4
@@ -151,9 +158,9 @@ template <int T, int E> struct Geo {
 // ------------------------------------------------------------------ Gram
 // Zero the stage columns no chunk writes (padding factors past the loaded
 // segments), once per row.
-template <int T, int E>
+template <int T, int E, bool AUG>
 __device__ __forceinline__ void stage_clear(int f, char *stage) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     const int l = lane();
     if constexpr (E == PREC_FP32) {
         float *Ys = reinterpret_cast<float *>(stage);
@@ -175,11 +182,11 @@ __device__ __forceinline__ void stage_clear(int f, char *stage) {
 // Stage ratings k0 .. k0+nv-1 of the row starting at rs (nv <= 32): their
 // item indices and values to ibuf/rbuf, the gathered rows y_i of the fixed
 // factors to the stage (FP32: Ys[rating][factor]; 16-bit: Yt[factor][rating]),
-// with the rating in column f. Slots past nv hold zero rows. Ends with the
-// stage visible to the whole wave.
-template <int T, int E>
+// with the rating in column f (AUG). Slots past nv hold zero rows. Ends with
+// the stage visible to the whole wave.
+template <int T, int E, bool AUG>
 __device__ __forceinline__ void stage_chunk(const UpdateArgs &a, int64_t rs, int k0, int nv, char *lds) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     const int l = lane();
     const int f = a.f;
     int *ibuf = reinterpret_cast<int *>(lds);
@@ -197,15 +204,17 @@ __device__ __forceinline__ void stage_chunk(const UpdateArgs &a, int64_t rs, int
         int k = l / nseg, s = l % nseg;
         for (int task = l; task < CHUNK * nseg; task += WAVE) {
             const int id = ibuf[k];
-            const float *src = id >= 0 ? a.Y + (int64_t)id * G::FP + 4 * s : a.zero32 + 4 * s;
+            const float *src = id >= 0 ? a.Y + (int64_t)id * G::LD + 4 * s : a.zero32 + 4 * s;
             const f32x4 v = *reinterpret_cast<const f32x4 *>(src);
             *reinterpret_cast<f32x4 *>(Ys + k * G::YR + 4 * s) = v;
             k += dk;
             s += ds;
             if (s >= nseg) { s -= nseg; ++k; }
         }
-        wave_sync();
-        if (l < CHUNK) Ys[l * G::YR + f] = rbuf[l];
+        if constexpr (AUG) {
+            wave_sync();
+            if (l < CHUNK) Ys[l * G::YR + f] = rbuf[l];
+        }
     } else {
         uint16_t *Yt = reinterpret_cast<uint16_t *>(stage);
         const uint16_t *Ysh = a.Ys;
@@ -221,7 +230,7 @@ __device__ __forceinline__ void stage_chunk(const UpdateArgs &a, int64_t rs, int
                 // Unused slots of the last chunk read a row of zeros: the
                 // load itself is unconditional.
                 const int id = ibuf[8 * g + e];
-                const uint16_t *src = id >= 0 ? Ysh + (int64_t)id * G::FP + 8 * s : a.zero16 + 8 * s;
+                const uint16_t *src = id >= 0 ? Ysh + (int64_t)id * G::LD + 8 * s : a.zero16 + 8 * s;
                 d[e] = *reinterpret_cast<const u32x4 *>(src);
             }
 #pragma unroll
@@ -237,13 +246,37 @@ __device__ __forceinline__ void stage_chunk(const UpdateArgs &a, int64_t rs, int
                 *reinterpret_cast<u32x4 *>(Yt + G::yt_row(8 * s + 2 * v + 1) * G::YT_H + 8 * g) = hi;
             }
         }
-        wave_sync();
-        if (l < CHUNK) Yt[G::yt_row(f) * G::YT_H + l] = to16<E>(rbuf[l]);
+        if constexpr (AUG) {
+            wave_sync();
+            if (l < CHUNK) Yt[G::yt_row(f) * G::YT_H + l] = to16<E>(rbuf[l]);
+        }
     }
     wave_sync();
 }
 
-// Accumulates the lower tiles of the augmented Gram of one row into acc
+// b without a rating column (f = 16T, where a column for the rating would
+// take another block of tiles): lane (q, c) holds the 16-bit ratings of its
+// operand rows 8q .. 8q+7 and adds their products with its column's entries,
+// bc[I] += sum_j Y[8q + j][16I + c] r[8q + j], FP32 sums. The four q's sums
+// are added when the row's Gram is done.
+template <int T, int E>
+__device__ __forceinline__ void rating_dots(const u32x4 (&F)[T], const u32x4 &R, float (&bc)[T]) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+    for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int I = 0; I < T; ++I) {
+            if constexpr (E == PREC_BF16)
+                bc[I] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, (uint32_t)F[I][w]),
+                                                        __builtin_bit_cast(b2, (uint32_t)R[w]), bc[I], false);
+            else
+                bc[I] = __builtin_amdgcn_fdot2(__builtin_bit_cast(h2, (uint32_t)F[I][w]),
+                                               __builtin_bit_cast(h2, (uint32_t)R[w]), bc[I], false);
+        }
+}
+
+// Accumulates the lower tiles of the (AUG: augmented) Gram of one row into acc
 // (q = lane/16, c = lane%16): diagonal tiles in the MFMA accumulator layout,
 // acc[tile_id(I,I)][r] = G[16I + 4q + r][16I + c]; off-diagonal tiles as
 // the accumulator of the transposed product, acc[tile_id(I,J)][r] =
@@ -261,17 +294,18 @@ __device__ __forceinline__ void stage_chunk(const UpdateArgs &a, int64_t rs, int
 // lane i supplies the address of 4 halves, Yr[8q + 4h + i/4][16I + 4(i%4)
 // .. +3], and lane j receives element j + 16t of the group's 64, which is
 // Yr[8q + 4h + t][16I + j], t = 0..3.
-template <int T, int E>
+template <int T, int E, bool AUG>
 __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs, int n,
-                                                 f32x4 (&acc)[Geo<T, E>::NT], char *lds) {
-    using G = Geo<T, E>;
+                                                 f32x4 (&acc)[T * (T + 1) / 2], float (&bc)[T], char *lds) {
+    using G = Geo<T, E, AUG>;
     constexpr int RS = G::RS16;
     typedef short v4i16 __attribute__((ext_vector_type(4)));
     typedef __attribute__((address_space(3))) v4i16 lds_v4i16;
     const int l = lane();
-    const int f = a.f;
+    const int f = AUG ? a.f : G::FP;
     int *ibuf = reinterpret_cast<int *>(lds);
     float *rbuf = reinterpret_cast<float *>(lds) + 32;
+    uint16_t *rb16 = reinterpret_cast<uint16_t *>(rbuf);  // the ratings in 16 bits instead (AUG = false)
     uint16_t *Yr = reinterpret_cast<uint16_t *>(lds + G::MISC_FLOATS * 4);
     const int nseg = (f + 7) >> 3;
     const bool active = l < 4 * nseg;  // task (g, s) of lane l
@@ -288,8 +322,9 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
     // column f, which each chunk writes (when f % 8 != 0 it lies in the last
     // gathered segment, whose padding halves are zero in the shadow rows)
     // (in 16-byte pieces: piece e is row e % 32, columns 8 nseg + 8 (e / 32))
-    for (int e = l; e < 4 * (G::FP - 8 * nseg); e += WAVE)
-        *reinterpret_cast<u32x4 *>(Yr + (e & 31) * RS + 8 * nseg + 8 * (e >> 5)) = u32x4{0u, 0u, 0u, 0u};
+    if constexpr (AUG)
+        for (int e = l; e < 4 * (G::FP - 8 * nseg); e += WAVE)
+            *reinterpret_cast<u32x4 *>(Yr + (e & 31) * RS + 8 * nseg + 8 * (e >> 5)) = u32x4{0u, 0u, 0u, 0u};
     // Raw indices and ratings of the chunk at k0, loaded by every lane (lane
     // l and l + 32 alike) at positions clamped into the row, so the loads
     // are unconditional; the positions past the row's end are masked when
@@ -307,7 +342,8 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
         const int l31 = lane_here() & 31;
         const bool in = k0 + l31 < n;
         ibuf[l31] = in ? id_raw : -1;
-        rbuf[l31] = in ? v_raw : 0.f;
+        if constexpr (AUG) rbuf[l31] = in ? v_raw : 0.f;
+        else rb16[l31] = in ? to16<E>(v_raw) : (uint16_t)0;
         wave_sync();
         if (active) {
             // the task's eight indices in two 16-byte reads, so the loads
@@ -318,16 +354,16 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
             const int ids[8] = {i0.x, i0.y, i0.z, i0.w, i1.x, i1.y, i1.z, i1.w};
             if (a.ys_bytes > 0) {
                 // Buffer loads with a 32-bit byte offset: a slot past the
-                // row's end (id -1) has an offset of 2^32 - 2 FP + 2 soff,
+                // row's end (id -1) has an offset of 2^32 - 2 LD + 2 soff,
                 // beyond the buffer, and reads zeros.
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     d[e] = __builtin_bit_cast(
-                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(ysr, ids[e] * (2 * G::FP) + soff2, 0, 0));
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(ysr, ids[e] * (2 * G::LD) + soff2, 0, 0));
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const uint16_t *src = (ids[e] >= 0 ? a.Ys + (int64_t)ids[e] * G::FP : a.zero16) + soff;
+                    const uint16_t *src = (ids[e] >= 0 ? a.Ys + (int64_t)ids[e] * G::LD : a.zero16) + soff;
                     d[e] = *reinterpret_cast<const u32x4 *>(src);
                 }
             }
@@ -343,8 +379,12 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
 #pragma unroll
             for (int e = 0; e < 8; ++e) *reinterpret_cast<u32x4 *>(wbase + e * RS) = d[e];
         }
-        if (const int lh = lane_here(); lh < CHUNK) Yr[lh * RS + f] = to16<E>(rbuf[lh]);
+        if constexpr (AUG) {
+            if (const int lh = lane_here(); lh < CHUNK) Yr[lh * RS + f] = to16<E>(rbuf[lh]);
+        }
         wave_sync();
+        u32x4 R;  // the ratings of this lane's operand rows
+        if constexpr (!AUG) R = *reinterpret_cast<const u32x4 *>(rb16 + 8 * (l >> 4));
         u32x4 F[T];
 #pragma unroll
         for (int I = 0; I < T; ++I) {
@@ -360,6 +400,7 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
             gather(k0 + CHUNK, nid, nval);
             load_ids(k0 + 2 * CHUNK, nid, nval);
         }
+        if constexpr (!AUG) rating_dots<T, E>(F, R, bc);
 #pragma unroll
         for (int I = 0; I < T; ++I)
 #pragma unroll
@@ -400,12 +441,17 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
 // done. Index and rating loads past the row's end read its last rating.
 // The loop of gram_row16_dma, with the two stage buffers and the two index /
 // rating buffer pairs as distinct pointers.
-template <int T, int E>
-__device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, int n, f32x4 (&acc)[Geo<T, E>::NT],
+// T % 4 == 0: a stage row is a multiple of 128 bytes, and the four rows of a
+// transposing read would share LDS banks; column block I of row k is kept at
+// block I ^ (k % 4) instead (the lane that fills a slot loads that slot's
+// column, the operand reads of block I take I ^ (their row % 4)).
+template <int T, int E, bool AUG>
+__device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, int n,
+                                              f32x4 (&acc)[T * (T + 1) / 2], float (&bc)[T],
                                               uint16_t *__restrict__ buf0, uint16_t *__restrict__ buf1,
                                               int *__restrict__ ib0, int *__restrict__ ib1,
                                               float *__restrict__ rb0, float *__restrict__ rb1) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     constexpr int RS = G::FP;             // stage row stride, halves
     constexpr int NS = 2 * T;             // 16-byte segments per row
     typedef short v4i16 __attribute__((ext_vector_type(4)));
@@ -414,9 +460,13 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
     const int l = lane();
     const int f = a.f;
     const bool active = l < 4 * NS;
+    constexpr bool SWZ = T % 4 == 0;
     const int g = l / NS, s = l - g * NS;
-    const int soff2 = 16 * s;
-    const int roff = (8 * (l >> 4) + ((l & 15) >> 2)) * RS + 4 * (l & 3);
+    const int soff2 = 16 * (SWZ ? s ^ (2 * (g & 3)) : s);  // row 4e + g of the chunk: row % 4 = g % 4
+    const int rrow = (8 * (l >> 4) + ((l & 15) >> 2)) * RS + 4 * (l & 3);
+    int roff[SWZ ? 4 : 1];  // block I at roff[I % 4] + 16 * (I - I % 4); without the permutation roff[0] + 16 I
+#pragma unroll
+    for (int b = 0; b < (SWZ ? 4 : 1); ++b) roff[b] = rrow + (SWZ ? 16 * (b ^ ((l & 15) >> 2)) : 0);
     const int nch = (n + CHUNK - 1) / CHUNK;
     const __amdgpu_buffer_rsrc_t ysr =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(a.Ys), (short)0, a.ys_bytes, 0x00020000);
@@ -439,7 +489,8 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
         const int m = lane_here() & 31;
         const bool in = CHUNK * j + m < n;
         ib[8 * (m & 3) + (m >> 2)] = in ? id_raw : -1;
-        rb[m] = in ? v_raw : 0.f;
+        if constexpr (AUG) rb[m] = in ? v_raw : 0.f;
+        else reinterpret_cast<uint16_t *>(rb)[m] = in ? to16<E>(v_raw) : (uint16_t)0;
     };
     // D(j) (parity P): the eight LDS-DMA loads of chunk j into buffer P
     auto dma = [&](auto parity) {
@@ -455,7 +506,7 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
 #pragma unroll
             for (int e = 0; e < 8; ++e)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(ysr, (lds_void *)(dst + 4 * e * RS), 16,
-                                                         ids[e] * (2 * G::FP) + soff2, 0, 0, 0);
+                                                         ids[e] * (2 * G::LD) + soff2, 0, 0, 0);
         }
     };
     using P0 = std::integral_constant<int, 0>;
@@ -487,13 +538,18 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
             for (int p = l; p < (CHUNK - nv) * NS; p += WAVE)
                 *reinterpret_cast<u32x4 *>(buf + (nv + p / NS) * RS + 8 * (p % NS)) = u32x4{0u, 0u, 0u, 0u};
         }
-        if (const int lh = lane_here(); lh < CHUNK) buf[lh * RS + f] = to16<E>(rb[lh]);
+        if constexpr (AUG) {
+            if (const int lh = lane_here(); lh < CHUNK) buf[lh * RS + f] = to16<E>(rb[lh]);
+        }
         wave_sync();
+        u32x4 R;  // the ratings of this lane's operand rows
+        if constexpr (!AUG) R = *reinterpret_cast<const u32x4 *>(reinterpret_cast<const uint16_t *>(rb) + 8 * (l >> 4));
         u32x4 F[T];
 #pragma unroll
         for (int I = 0; I < T; ++I) {
-            const v4i16 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)(buf + roff + 16 * I));
-            const v4i16 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)(buf + roff + 4 * RS + 16 * I));
+            uint16_t *src = buf + roff[SWZ ? I % 4 : 0] + 16 * (SWZ ? I - I % 4 : I);
+            const v4i16 t0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)src);
+            const v4i16 t1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4i16 *)(src + 4 * RS));
             const u32x2 w0 = __builtin_bit_cast(u32x2, t0), w1 = __builtin_bit_cast(u32x2, t1);
             F[I] = u32x4{w0[0], w0[1], w1[0], w1[1]};
         }
@@ -504,6 +560,7 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
         dma(parity);
         if constexpr (P == 0) load_ids(k + 4, id0, v0);
         else load_ids(k + 4, id1, v1);
+        if constexpr (!AUG) rating_dots<T, E>(F, R, bc);
 #pragma unroll
         for (int I = 0; I < T; ++I)
 #pragma unroll
@@ -528,50 +585,58 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int T, int E>
+template <int T, int E, bool AUG>
 __device__ __forceinline__ void gram_row16_dma(const UpdateArgs &a, int64_t rs, int n,
-                                               f32x4 (&acc)[Geo<T, E>::NT], char *lds) {
-    using G = Geo<T, E>;
+                                               f32x4 (&acc)[T * (T + 1) / 2], float (&bc)[T], char *lds) {
+    using G = Geo<T, E, AUG>;
     constexpr int BUF = CHUNK * G::FP;  // halves per buffer
     if (n <= 0) return;
     uint16_t *stage = reinterpret_cast<uint16_t *>(lds + G::MISC_FLOATS * 4);
-    gram_dma_loop<T, E>(a, rs, n, acc, stage, stage + BUF, reinterpret_cast<int *>(lds),
+    gram_dma_loop<T, E, AUG>(a, rs, n, acc, bc, stage, stage + BUF, reinterpret_cast<int *>(lds),
                         reinterpret_cast<int *>(stage + 2 * BUF), reinterpret_cast<float *>(lds) + 32,
                         reinterpret_cast<float *>(stage + 2 * BUF) + 32);
 }
 
-template <int T, int E>
-__device__ __forceinline__ void gram_row(const UpdateArgs &a, int64_t rs, int n,
-                                         f32x4 (&acc)[Geo<T, E>::NT], char *lds) {
-    using G = Geo<T, E>;
+// The Gram of ratings rs .. rs + n - 1 of a row; with AUG = false also b, in
+// column form, each lane row q holding its share of the ratings (q4_sum adds
+// them). With AUG, b is row f of the tiles.
+template <int T, int E, bool AUG>
+__device__ __forceinline__ void gram_row(const UpdateArgs &a, int64_t rs, int n, f32x4 (&acc)[T * (T + 1) / 2],
+                                         float (&bc)[T], char *lds) {
+    using G = Geo<T, E, AUG>;
     const int l = lane();
     char *stage = lds + G::MISC_FLOATS * 4;
 #pragma unroll
     for (int t = 0; t < G::NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int I = 0; I < T; ++I) bc[I] = 0.f;
     if constexpr (G::DMA_GRAM) {
         if (a.ys_bytes > 0 && a.gram_dma) {
-            gram_row16_dma<T, E>(a, rs, n, acc, lds);
+            gram_row16_dma<T, E, AUG>(a, rs, n, acc, bc, lds);
             return;
         }
     }
-    if constexpr (E != PREC_FP32 && T <= 9) {
-        // f <= 128: at most 16 segments, one task per lane (every f of
-        // T <= 8; f = 128 of T = 9, whose rating column is the 129th)
-        if (T <= 8 || a.f <= 128) {
-            gram_row16_piped<T, E>(a, rs, n, acc, lds);
-            return;
-        }
+    if constexpr (E != PREC_FP32 && T <= 8) {
+        // f <= 128: at most 16 segments, one task per lane
+        gram_row16_piped<T, E, AUG>(a, rs, n, acc, bc, lds);
+        return;
     }
-    stage_clear<T, E>(a.f, stage);
+    if constexpr (AUG) stage_clear<T, E, AUG>(a.f, stage);
     for (int k0 = 0; k0 < n; k0 += CHUNK) {
-        stage_chunk<T, E>(a, rs, k0, min(CHUNK, n - k0), lds);
+        stage_chunk<T, E, AUG>(a, rs, k0, min(CHUNK, n - k0), lds);
         if constexpr (E == PREC_FP32) {
             const float *Ys = reinterpret_cast<const float *>(stage);
+            const float *rbuf = reinterpret_cast<const float *>(lds) + 32;
 #pragma unroll
             for (int ks = 0; ks < CHUNK / 4; ++ks) {
                 float F[T];
 #pragma unroll
                 for (int I = 0; I < T; ++I) F[I] = Ys[(4 * ks + (l >> 4)) * G::YR + 16 * I + (l & 15)];
+                if constexpr (!AUG) {
+                    const float r = rbuf[4 * ks + (l >> 4)];
+#pragma unroll
+                    for (int I = 0; I < T; ++I) bc[I] = fmaf(F[I], r, bc[I]);
+                }
 #pragma unroll
                 for (int I = 0; I < T; ++I)
 #pragma unroll
@@ -858,18 +923,30 @@ __device__ __forceinline__ void split16(const f32x4 &x, f16x4 &hi, f16x4 &lo) {
 //                  kept to ~2^-22 relative; the entries of L are bounded by
 //                  sqrt(A_ii), inside FP16's range for the ratings
 //                  als_set_train accepts)
-// The last block holds row f (the augmented row, never a pivot): yl gets
+// AUG: the last block holds row f (the augmented row, never a pivot): yl gets
 // its reduced entries (row form) just before that block is factored.
-template <int T, int K, int NT, bool SPLIT>
-__device__ __forceinline__ void chol_panels(f32x4 (&a)[NT], int f, f32x4 &yl) {
+// Otherwise every block is full and the forward substitution runs beside the
+// factorisation on b itself: bc (column form) holds b in row q = 0 and, from
+// panel 0 on, minus this lane row's share of the finished blocks' terms in
+// every q, so that block K's right-hand side is its sum over the q when its
+// turn comes: z_K = W_KK (b_K - sum_J L_KJ z_J), kept in zr (row form).
+template <int T, int K, int NT, bool SPLIT, bool AUG>
+__device__ __forceinline__ void chol_panels(f32x4 (&a)[NT], int f, f32x4 &yl, float (&bc)[T], f32x4 (&zr)[T]) {
     if constexpr (K < T) {
         const int jend = min(16, f - 16 * K);
-        if constexpr (K == T - 1) {
+        if constexpr (AUG && K == T - 1) {
             const int l = lane();
 #pragma unroll
             for (int r = 0; r < 4; ++r) yl[r] = __shfl(a[tile_id(K, K)][r], (l & 48) | (f & 15), WAVE);
         }
-        diag_factor<(K + 1 < T)>(a[tile_id(K, K)], jend);
+        diag_factor<(!AUG || K + 1 < T)>(a[tile_id(K, K)], jend);
+        if constexpr (!AUG) {
+            const f32x4 tr = col_to_row(q4_sum(bc[K]));
+            float u = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u += a[tile_id(K, K)][r] * tr[r];
+            zr[K] = col_to_row(q4_sum(u));
+        }
         if constexpr (K + 1 < T) {
 #pragma unroll
             for (int I = K + 1; I < T; ++I) {
@@ -879,6 +956,12 @@ __device__ __forceinline__ void chol_panels(f32x4 (&a)[NT], int f, f32x4 &yl) {
                 for (int r = 0; r < 4; ++r)
                     nw = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tile_id(K, K)][r], o[r], nw, 0, 0, 0);
                 a[tile_id(I, K)] = nw;
+            }
+            if constexpr (!AUG) {
+#pragma unroll
+                for (int I = K + 1; I < T; ++I)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bc[I] -= a[tile_id(I, K)][r] * zr[K][r];
             }
             if constexpr (SPLIT) {
                 // Each panel tile as [hi | lo], the 8 halves a lane feeds a
@@ -920,19 +1003,24 @@ __device__ __forceinline__ void chol_panels(f32x4 (&a)[NT], int f, f32x4 &yl) {
                     }
             }
         }
-        chol_panels<T, K + 1, NT, SPLIT>(a, f, yl);
+        chol_panels<T, K + 1, NT, SPLIT, AUG>(a, f, yl, bc, zr);
     }
 }
 
-// Factorises the augmented matrix in place and returns z = L^-1 b in row
-// form (zero past f). A pivot <= 0 leaves non-finite values that reach x
+// Factorises the matrix in place and returns z = L^-1 b in row form (zero past
+// f); b is row f of the tiles (AUG) or bc, in column form (used up). A pivot <= 0 leaves non-finite values that reach x
 // (the caller checks x); the return value is kept for that interface.
 // SPLIT: the trailing updates on FP16 hi/lo parts (chol_panels).
-template <int T, int NT, bool SPLIT = false>
-__device__ __forceinline__ bool chol_regs(f32x4 (&a)[NT], int f, f32x4 (&zr)[T]) {
-    f32x4 yl;
-    chol_panels<T, 0, NT, SPLIT>(a, f, yl);
+template <int T, int NT, bool SPLIT, bool AUG>
+__device__ __forceinline__ bool chol_regs(f32x4 (&a)[NT], int f, float (&bc)[T], f32x4 (&zr)[T]) {
     const int l = lane(), q = l >> 4, c = l & 15;
+    f32x4 yl;
+    if constexpr (!AUG) {
+#pragma unroll
+        for (int K = 0; K < T; ++K) bc[K] = q == 0 ? bc[K] : 0.f;
+    }
+    chol_panels<T, 0, NT, SPLIT, AUG>(a, f, yl, bc, zr);
+    if constexpr (!AUG) return true;
 #pragma unroll
     for (int K = 0; K + 1 < T; ++K)
 #pragma unroll
@@ -1042,14 +1130,16 @@ __device__ __forceinline__ double rows16_scatter_d(const double (&v)[4]) {
 // discarded entry f. x0 in column form (zero past f); xs (16T floats of LDS)
 // holds it in memory order, where the row form of a block is one 16-byte
 // read. The last diagonal tile keeps its row and column f symmetric.
-template <int T, int NT>
-__device__ __forceinline__ void warm_row_f(f32x4 (&a)[NT], int f, const float (&xc)[T], float *xs, float *bs) {
+// Without the augmented row (AUG = false) bc holds b and takes r0.
+template <int T, int NT, bool AUG>
+__device__ __forceinline__ void warm_row_f(f32x4 (&a)[NT], int f, const float (&xc)[T], float *xs, float *bs,
+                                           float (&bc)[T]) {
     const int l = lane(), q = l >> 4, c = l & 15, fr = f & 15;
     if (l < 16) {
 #pragma unroll
         for (int J = 0; J < T; ++J) xs[16 * J + l] = xc[J];
     }
-    if (c == fr) {
+    if (AUG && c == fr) {
         // lane (q, f % 16) holds b[16K + 4q + r] in register r of tile (T-1, K)
 #pragma unroll
         for (int K = 0; K < T; ++K) *reinterpret_cast<f32x4 *>(bs + 16 * K + 4 * q) = a[tile_id(T - 1, K)];
@@ -1073,6 +1163,10 @@ __device__ __forceinline__ void warm_row_f(f32x4 (&a)[NT], int f, const float (&
         // lane (c / 4, c), which holds the total for register c % 4 of row c / 4
         const double rs = (K + 1 < T) ? rows16_scatter_d(rp) : 0.0;
         const double y = q4_sum_d(cp) + __shfl(rs, ((c >> 2) << 4) | c, WAVE);
+        if constexpr (!AUG) {
+            bc[K] = (float)((double)bc[K] - y);
+            continue;
+        }
         const float resc = (16 * K + c < f) ? (float)((double)bs[16 * K + c] - y) : 0.f;
         const f32x4 res = col_to_row(resc);  // lane (q, c): r0[16K + 4q + r]
         if (K + 1 < T) {
@@ -1091,9 +1185,9 @@ __device__ __forceinline__ void warm_row_f(f32x4 (&a)[NT], int f, const float (&
 }
 
 // Residual from this wave's scratch copy Ag of the augmented tiles, taken
-// before the factorisation (row f holds b). x column form; r column form
-// (zero past f).
-template <int T>
+// before the factorisation (row f holds b; AUG = false: b follows the tiles).
+// x column form; r column form (zero past f).
+template <int T, bool AUG>
 __device__ __forceinline__ void residual_copy(const float *Ag, int f, const float (&xc)[T], float (&rc)[T]) {
     const int l = lane(), q = l >> 4;
     f32x4 xr[T];
@@ -1123,7 +1217,8 @@ __device__ __forceinline__ void residual_copy(const float *Ag, int f, const floa
         }
         const double cs = q4_sum_d(cp);
         // b_K in row form: lane (q, f & 15) of tile (T-1, K), register r.
-        const f32x4 br = *reinterpret_cast<const f32x4 *>(Ag + tile_id(T - 1, K) * 256 + 4 * ((q << 4) | (f & 15)));
+        const f32x4 br = *reinterpret_cast<const f32x4 *>(
+            Ag + (AUG ? tile_id(T - 1, K) * 256 + 4 * ((q << 4) | (f & 15)) : T * (T + 1) / 2 * 256 + 16 * K + 4 * q));
         f32x4 res;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -1134,9 +1229,9 @@ __device__ __forceinline__ void residual_copy(const float *Ag, int f, const floa
     }
 }
 
-template <int T, int E>
+template <int T, int E, bool AUG>
 __device__ __forceinline__ float stage_at(const char *stage, int k, int j) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     if constexpr (E == PREC_FP32)
         return reinterpret_cast<const float *>(stage)[k * G::YR + j];
     else
@@ -1144,9 +1239,9 @@ __device__ __forceinline__ float stage_at(const char *stage, int k, int j) {
 }
 
 // r_j += sum_k y_k[j] e_k over the staged chunk, for factor j.
-template <int T, int E>
+template <int T, int E, bool AUG>
 __device__ __forceinline__ double stage_row_dot(const char *stage, int j, const double *eb) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     double acc = 0.0;
     if constexpr (E == PREC_FP32) {
         const float *Ys = reinterpret_cast<const float *>(stage);
@@ -1184,10 +1279,10 @@ __device__ __forceinline__ void lanes_to_colform(const double (&acc)[NJ], int f,
 // restages the FP32 master rows, E = PREC_FP32, whatever the Gram's
 // precision), reg the FP32 lambda * n the diagonal got. Products and sums in
 // FP64. x column form; r column form (zero past f).
-template <int T, int E>
+template <int T, int E, bool AUG>
 __device__ __forceinline__ void residual_mf(const UpdateArgs &a, int64_t rs, int n, float reg, const float (&xc)[T],
                                             float (&rc)[T], char *lds) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     constexpr int NJ = (G::FP + WAVE - 1) / WAVE;
     constexpr int HALF = G::FP / 2;
     const int l = lane(), f = a.f;
@@ -1206,10 +1301,10 @@ __device__ __forceinline__ void residual_mf(const UpdateArgs &a, int64_t rs, int
     for (int m = 0; m < NJ; ++m) acc[m] = 0.0;
     for (int k0 = 0; k0 < n; k0 += CHUNK) {
         const int nv = min(CHUNK, n - k0);
-        stage_chunk<T, E>(a, rs, k0, nv, lds);
+        stage_chunk<T, E, AUG>(a, rs, k0, nv, lds);
         // e_k = r_k - y_k . x: lane (k, half) sums the factors [jb, je)
         double dot = 0.0;
-        for (int j = jb; j < je; ++j) dot += (double)stage_at<T, E>(stage, k, j) * (double)xs[j];
+        for (int j = jb; j < je; ++j) dot += (double)stage_at<T, E, AUG>(stage, k, j) * (double)xs[j];
         dot = halves_sum_d(dot);
         if (l < CHUNK) {
             float rk = rbuf[k];
@@ -1219,7 +1314,7 @@ __device__ __forceinline__ void residual_mf(const UpdateArgs &a, int64_t rs, int
         wave_sync();
 #pragma unroll
         for (int m = 0; m < NJ; ++m)
-            if (WAVE * m + l < f) acc[m] += stage_row_dot<T, E>(stage, WAVE * m + l, eb);
+            if (WAVE * m + l < f) acc[m] += stage_row_dot<T, E, AUG>(stage, WAVE * m + l, eb);
         wave_sync();
     }
     lanes_to_colform<T, 0>(acc, f, reg, xc, rc);
@@ -1313,19 +1408,20 @@ __device__ __forceinline__ void cg_regs(const f32x4 (&A)[NT], int f, const float
     }
 }
 
-// Column-form vector -> one row of a 16T-strided matrix in global memory
-// (row-group q stores blocks q, q+4, ...; 16 consecutive floats each).
-template <int T>
+// Column-form vector -> one row of a factor matrix in global memory
+// (row-group q stores blocks q, q+4, ...; 16 consecutive floats each). PAD:
+// a block of zeros follows (the matrices' stride is the augmented system's).
+template <int T, bool PAD = false>
 __device__ __forceinline__ void store_colform(float *dst, const float (&v)[T]) {
     const int l = lane(), q = l >> 4, c = l & 15;
 #pragma unroll
-    for (int J4 = 0; J4 < T; J4 += 4) {
+    for (int J4 = 0; J4 < T + PAD; J4 += 4) {
         const int J = J4 + q;
         float val = 0.f;
 #pragma unroll
         for (int k = 0; k < 4; ++k)
             if (J4 + k < T && q == k) val = v[J4 + k];
-        if (J < T) dst[16 * J + c] = val;
+        if (J < T + PAD) dst[16 * J + c] = val;
     }
 }
 template <int T, int E>
@@ -1412,10 +1508,10 @@ __device__ __forceinline__ float rows16_scatter4(const float (&v)[4]) {
 // one 16x16x32 MFMA per tile. FP32 rows: 4 factors, four 16x16x4 MFMAs,
 // the j-th taking factor 4 (4s + q) + j as its k = q (the contraction over
 // the factors runs in any order, the same for both operands).
-template <int TD, int T, int E>
+template <int TD, int T, int E, bool AUG>
 __device__ __forceinline__ void dual_operands(const UpdateArgs &a, const int (&id)[TD], int s, int nseg,
                                               u32x4 (&F)[TD]) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     const int seg = 4 * s + (lane() >> 4);
     constexpr int SEGW = E == PREC_FP32 ? 4 : 8;  // elements per 16-byte segment
 #pragma unroll
@@ -1423,9 +1519,9 @@ __device__ __forceinline__ void dual_operands(const UpdateArgs &a, const int (&i
         F[I] = u32x4{0u, 0u, 0u, 0u};
         if (id[I] >= 0 && seg < nseg) {
             if constexpr (E == PREC_FP32)
-                F[I] = *reinterpret_cast<const u32x4 *>(a.Y + (int64_t)id[I] * G::FP + SEGW * seg);
+                F[I] = *reinterpret_cast<const u32x4 *>(a.Y + (int64_t)id[I] * G::LD + SEGW * seg);
             else
-                F[I] = *reinterpret_cast<const u32x4 *>(a.Ys + (int64_t)id[I] * G::FP + SEGW * seg);
+                F[I] = *reinterpret_cast<const u32x4 *>(a.Ys + (int64_t)id[I] * G::LD + SEGW * seg);
         }
     }
 }
@@ -1437,7 +1533,7 @@ __device__ __forceinline__ void dual_operands(const UpdateArgs &a, const int (&i
 // stays far below the rounding of the 16-bit Gram that every row of the
 // mixed path carries; no refinement step is taken here.
 // xs: 16T floats of this wave's LDS.
-template <int TD, int T, int E>
+template <int TD, int T, int E, bool AUG>
 __device__ __forceinline__ void dual_row(const UpdateArgs &a, int64_t rs, int n, float reg, float (&xc)[T],
                                          float *xs) {
     constexpr int NTD = TD * (TD + 1) / 2;
@@ -1465,7 +1561,7 @@ __device__ __forceinline__ void dual_row(const UpdateArgs &a, int64_t rs, int n,
     for (int t = 0; t < NTD; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < ks; ++s) {
         u32x4 F[TD];
-        dual_operands<TD, T, E>(a, id, s, nseg, F);
+        dual_operands<TD, T, E, AUG>(a, id, s, nseg, F);
 #pragma unroll
         for (int I = 0; I < TD; ++I)
 #pragma unroll
@@ -1505,15 +1601,15 @@ __device__ __forceinline__ void dual_row(const UpdateArgs &a, int64_t rs, int n,
         }
     }
     f32x4 zr[TD];
-    chol_regs<TD, NTD, (E != PREC_FP32)>(acc, n, zr);
     float al[TD];
+    chol_regs<TD, NTD, (E != PREC_FP32), true>(acc, n, al, zr);
     back_solve<TD>(acc, n, zr, al);
     // x = Y^T alpha: lane (q, c) multiplies segment 4s + q of row 16I + c by
     // alpha[16I + c]; after the scattered sum over c, lane c holds factor
     // 8 (4s + q) + c / 2 (16-bit) or 4 (4s + q) + c % 4 (FP32).
     for (int s = 0; s < ks; ++s) {
         u32x4 F[TD];
-        dual_operands<TD, T, E>(a, id, s, nseg, F);
+        dual_operands<TD, T, E, AUG>(a, id, s, nseg, F);
         const int seg = 4 * s + q;
         if constexpr (E == PREC_FP32) {
             float p[4] = {0.f, 0.f, 0.f, 0.f};
@@ -1543,24 +1639,24 @@ __device__ __forceinline__ void dual_row(const UpdateArgs &a, int64_t rs, int n,
 }
 
 // The dual system of the fewest tiles that hold n + 1 rows.
-template <int TD, int TDMAX, int T, int E>
+template <int TD, int TDMAX, int T, int E, bool AUG>
 __device__ __forceinline__ void dual_pick(const UpdateArgs &a, int64_t rs, int n, float reg, float (&xc)[T],
                                           float *xs) {
     if constexpr (TD < TDMAX) {
-        if (n < 16 * TD) dual_row<TD, T, E>(a, rs, n, reg, xc, xs);
-        else dual_pick<TD + 1, TDMAX, T, E>(a, rs, n, reg, xc, xs);
+        if (n < 16 * TD) dual_row<TD, T, E, AUG>(a, rs, n, reg, xc, xs);
+        else dual_pick<TD + 1, TDMAX, T, E, AUG>(a, rs, n, reg, xc, xs);
     } else {
-        dual_row<TD, T, E>(a, rs, n, reg, xc, xs);
+        dual_row<TD, T, E, AUG>(a, rs, n, reg, xc, xs);
     }
 }
 
 // Every work unit of queue batch b of one model.
-template <int T, int E, int S>
+template <int T, int E, int S, bool AUG>
 __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     const int l = lane();
     const int f = a.f;
-    float *Ascr = a.scratch ? a.scratch + (int64_t)blockIdx.x * G::NT * 256 : nullptr;
+    float *Ascr = a.scratch ? a.scratch + (int64_t)blockIdx.x * G::PART : nullptr;
     f32x4 acc[G::NT];
     {
         const int u0 = a.batch_begin[b], u1 = a.batch_begin[b + 1];
@@ -1585,19 +1681,25 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
             float *xs = reinterpret_cast<float *>(lds) + 64;
             if constexpr (WARM_KERNEL) {
                 if (warm_row && l < G::FP / 4)
-                    __builtin_amdgcn_global_load_lds(a.X + (int64_t)row * G::FP + 4 * l,
+                    __builtin_amdgcn_global_load_lds(a.X + (int64_t)row * G::LD + 4 * l,
                                                      (__attribute__((address_space(3))) void *)xs, 16, 0, 0);
             }
             if (n > 0) {
-                gram_row<T, E>(a, w.y, w.z - w.y, acc, lds);
+                float bv[T];  // b, column form (AUG = false)
+                gram_row<T, E, AUG>(a, w.y, w.z - w.y, acc, bv, lds);
+                if constexpr (!AUG) {
+#pragma unroll
+                    for (int J = 0; J < T; ++J) bv[J] = q4_sum(bv[J]);
+                }
                 if (w.w >= 0) {
                     // Split row: publish this part's tiles; the last part to
                     // arrive sums every part in slot order and solves.
                     const int4 sp = a.splits[w.w];
                     const int part = (w.y - a.ptr[row]) / sp.z;
-                    float *mine = a.partial + (int64_t)(sp.x + part) * G::NT * 256;
+                    float *mine = a.partial + (int64_t)(sp.x + part) * G::PART;
 #pragma unroll
                     for (int t = 0; t < G::NT; ++t) *reinterpret_cast<f32x4 *>(mine + t * 256 + 4 * l) = acc[t];
+                    if constexpr (!AUG) store_colform<T>(mine + G::NT * 256, bv);
                     __threadfence();
                     int ticket = 0;
                     if (l == 0) ticket = atomicAdd(a.counters + w.w, 1);
@@ -1606,8 +1708,16 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                     __threadfence();
 #pragma unroll
                     for (int t = 0; t < G::NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if constexpr (!AUG) {
+#pragma unroll
+                        for (int J = 0; J < T; ++J) bv[J] = 0.f;
+                    }
                     for (int p = 0; p < sp.y; ++p) {
-                        const float *src = a.partial + (int64_t)(sp.x + p) * G::NT * 256;
+                        const float *src = a.partial + (int64_t)(sp.x + p) * G::PART;
+                        if constexpr (!AUG) {
+#pragma unroll
+                            for (int J = 0; J < T; ++J) bv[J] += src[G::NT * 256 + 16 * J + (l & 15)];
+                        }
                         // T tiles' loads in flight before their adds (one
                         // register reused for every tile would wait for each
                         // load in turn)
@@ -1646,6 +1756,7 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
 #pragma unroll
                             for (int t = 0; t < G::NT; ++t)
                                 *reinterpret_cast<f32x4 *>(Ascr + t * 256 + 4 * l) = acc[t];
+                            if constexpr (!AUG) store_colform<T>(Ascr + G::NT * 256, bv);
                         }
                     }
                     if constexpr (S == SOLVE_CHOL_REFINE || S == SOLVE_CHOL_WARM) {
@@ -1656,20 +1767,21 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                                 load_colform<T>(xs, f, x0);
                             } else {
-                                load_colform<T>(a.X + (int64_t)row * G::FP, f, x0);
+                                load_colform<T>(a.X + (int64_t)row * G::LD, f, x0);
                             }
-                            warm_row_f<T>(acc, f, x0, xs, reinterpret_cast<float *>(lds + G::MISC_FLOATS * 4));
+                            warm_row_f<T, G::NT, AUG>(acc, f, x0, xs, reinterpret_cast<float *>(lds + G::MISC_FLOATS * 4),
+                                                      bv);
                         }
                     }
                     f32x4 zr[T];
                     // the 16-bit-Gram paths factor with split-FP16 trailing updates
-                    ok = chol_regs<T, G::NT, (E != PREC_FP32)>(acc, f, zr);
+                    ok = chol_regs<T, G::NT, (E != PREC_FP32), AUG>(acc, f, bv, zr);
                     back_solve<T>(acc, f, zr, x);
                     if (warm) {
                         // x0 again (not kept live across the factorisation): from
                         // xs, where the residual wrote the same values, or from X
                         if (warm_row) load_colform<T>(xs, f, x0);
-                        else load_colform<T>(a.X + (int64_t)row * G::FP, f, x0);
+                        else load_colform<T>(a.X + (int64_t)row * G::LD, f, x0);
 #pragma unroll
                         for (int J = 0; J < T; ++J) x[J] += x0[J];
                     }
@@ -1679,8 +1791,8 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                             // restaged from the FP32 master rows: the residual of the
                             // unrounded system, which the correction solves then
                             // converge to (the 16-bit Gram's factor preconditions them)
-                            if (restage) residual_mf<T, PREC_FP32>(a, w.y, n, reg, x, rc, lds);
-                            else residual_copy<T>(Ascr, f, x, rc);
+                            if (restage) residual_mf<T, PREC_FP32, AUG>(a, w.y, n, reg, x, rc, lds);
+                            else residual_copy<T, AUG>(Ascr, f, x, rc);
                             correct<T>(acc, f, rc, x);
                         }
                     }
@@ -1690,16 +1802,15 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                         for (int t = 0; t < G::NT; ++t) *reinterpret_cast<f32x4 *>(dst + t * 256 + 4 * l) = acc[t];
                     }
                 } else {
-                    float bvec[T];
-                    extract_b<T>(acc, f, bvec);
+                    if constexpr (AUG) extract_b<T>(acc, f, bv);
                     if (a.cg_fp16_a) {
 #pragma unroll
                         for (int t = 0; t < G::NT; ++t)
 #pragma unroll
                             for (int r = 0; r < 4; ++r) acc[t][r] = (float)(_Float16)acc[t][r];
                     }
-                    load_colform<T>(a.X + (int64_t)row * G::FP, f, x);
-                    cg_regs<T>(acc, f, bvec, x, a.cg_iters, a.cg_tol);
+                    load_colform<T>(a.X + (int64_t)row * G::LD, f, x);
+                    cg_regs<T>(acc, f, bv, x, a.cg_iters, a.cg_tol);
                 }
                 bool finite = true;
 #pragma unroll
@@ -1711,25 +1822,25 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                     for (int J = 0; J < T; ++J) x[J] = 0.f;
                 }
             }
-            store_colform<T>(a.X + (int64_t)row * G::FP, x);
+            store_colform<T, !AUG>(a.X + (int64_t)row * G::LD, x);
             if constexpr (E != PREC_FP32) {
-                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::FP, x);
+                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::LD, x);
             }
         }
     }
 }
 
-template <int T, int E, int S>
+template <int T, int E, int S, bool AUG>
 __device__ __forceinline__ void update_body(const UpdateArgs &a) {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     for (int b = blockIdx.x; b < a.nbatches; b = next_batch(a.queue, a.nbatches)) {
-        run_batch<T, E, S>(a, b, lds);
+        run_batch<T, E, S, AUG>(a, b, lds);
     }
 }
 
-template <int T, int E, int S>
+template <int T, int E, int S, bool AUG>
 __global__ __launch_bounds__(WAVE) void update_kernel(UpdateArgs a) {
-    update_body<T, E, S>(a);
+    update_body<T, E, S, AUG>(a);
 }
 
 // Light rows through the dual system: whole rows with fewer than
@@ -1739,9 +1850,9 @@ __global__ __launch_bounds__(WAVE) void update_kernel(UpdateArgs a) {
 // none of its code. Four waves per SIMD (128 VGPRs; at T = 8 and 9 one or
 // two registers spill): its row is mostly VALU work on few live registers,
 // and four waves run it faster than three (users half -1.8% at f = 100).
-template <int T, int E, int S>
+template <int T, int E, int S, bool AUG>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 4))) void dual_kernel(UpdateArgs a) {
-    using G = Geo<T, E>;
+    using G = Geo<T, E, AUG>;
     extern __shared__ __attribute__((aligned(16))) char lds[];
     const int l = lane();
     float *xs = reinterpret_cast<float *>(lds) + 64;
@@ -1755,7 +1866,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
             for (int J = 0; J < T; ++J) x[J] = 0.f;
             if (n > 0) {
                 const float reg = (a.lambda_rows ? a.lambda_rows[row] : a.lambda) * (float)n;
-                dual_pick<1, G::DUAL_TD, T, E>(a, a.ptr[row], n, reg, x, xs);
+                dual_pick<1, G::DUAL_TD, T, E, AUG>(a, a.ptr[row], n, reg, x, xs);
                 bool finite = true;
 #pragma unroll
                 for (int J = 0; J < T; ++J) finite = finite && isfinite(x[J]);
@@ -1765,9 +1876,9 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
                     for (int J = 0; J < T; ++J) x[J] = 0.f;
                 }
             }
-            store_colform<T>(a.X + (int64_t)row * G::FP, x);
+            store_colform<T, !AUG>(a.X + (int64_t)row * G::LD, x);
             if constexpr (E != PREC_FP32) {
-                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::FP, x);
+                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::LD, x);
             }
         }
     }
@@ -1776,9 +1887,9 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
 // The refinement variant holds the factor, the solution and the FP64
 // residual pieces at once; at two waves per SIMD it trades a small spill
 // for twice the latency hiding of the one-wave form.
-template <int T, int E, int S>
+template <int T, int E, int S, bool AUG>
 __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(2, 2))) void update_kernel_w2(UpdateArgs a) {
-    update_body<T, E, S>(a);
+    update_body<T, E, S, AUG>(a);
 }
 
 }  // namespace als

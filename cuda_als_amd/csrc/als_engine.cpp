@@ -217,7 +217,7 @@ int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t spl
     }
     if ((rc = dev_alloc(e, &s.units, sc.units.size())) || (rc = dev_alloc(e, &s.batch, sc.batch_begin.size())) ||
         (rc = dev_alloc(e, &s.splits, sc.splits.size())) || (rc = dev_alloc(e, &s.counters, sc.splits.size())) ||
-        (rc = dev_alloc(e, &s.partial, (size_t)sc.nslots * (e->T * (e->T + 1) / 2) * 256)))
+        (rc = dev_alloc(e, &s.partial, (size_t)sc.nslots * part_floats(e->cfg.f))))
         return rc;
     if (!sc.units.empty())
         HIPCHK(e, hipMemcpyAsync(s.units, sc.units.data(), sc.units.size() * sizeof(int4), hipMemcpyHostToDevice, e->stream));
@@ -322,17 +322,17 @@ int launch_schedule(als_engine *e, const Side &s, const float *Y, const uint16_t
         d.queue = e->queue + 2;
         HIPCHK(e, hipEventRecord(e->dual_fork, st));
         HIPCHK(e, hipStreamWaitEvent(e->dual_stream, e->dual_fork, 0));
-        HIPCHK(e, launch_update(e->T, e->prec, solve, var, a, ugrid, e->lds, st));
-        HIPCHK(e, launch_dual(e->T, e->prec, solve, d, dgrid, e->dual_lds, e->dual_stream));
+        HIPCHK(e, launch_update(e->cfg.f, e->prec, solve, var, a, ugrid, e->lds, st));
+        HIPCHK(e, launch_dual(e->cfg.f, e->prec, solve, d, dgrid, e->dual_lds, e->dual_stream));
         HIPCHK(e, hipEventRecord(e->dual_join, e->dual_stream));
         HIPCHK(e, hipStreamWaitEvent(st, e->dual_join, 0));
         return ALS_OK;
     }
-    if (s.nbatches > 0) HIPCHK(e, launch_update(e->T, e->prec, solve, var, a, ugrid, e->lds, st));
+    if (s.nbatches > 0) HIPCHK(e, launch_update(e->cfg.f, e->prec, solve, var, a, ugrid, e->lds, st));
     if (s.dnbatches > 0) {
         const UpdateArgs d = dual_args(s, a);
-        if (Lsave) HIPCHK(e, launch_update(e->T, e->prec, solve, var, d, std::min(umax, s.dnbatches), e->lds, st));
-        else HIPCHK(e, launch_dual(e->T, e->prec, solve, d, dgrid, e->dual_lds, st));
+        if (Lsave) HIPCHK(e, launch_update(e->cfg.f, e->prec, solve, var, d, std::min(umax, s.dnbatches), e->lds, st));
+        else HIPCHK(e, launch_dual(e->cfg.f, e->prec, solve, d, dgrid, e->dual_lds, st));
     }
     return ALS_OK;
 }
@@ -469,8 +469,8 @@ int als_create(const als_config *cfg, als_engine **out) {
     e->num_cu = prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&e->own_stream, hipStreamNonBlocking) != hipSuccess) { delete e; return ALS_E_HIP; }
     e->stream = e->own_stream;
-    e->lds = update_lds_bytes(e->T, e->prec, e->solve, cfg->refine_steps);
-    const void *k = update_kernel_ptr(e->T, e->prec, e->solve);
+    e->lds = update_lds_bytes(cfg->f, e->prec, e->solve);
+    const void *k = update_kernel_ptr(cfg->f, e->prec, e->solve);
     int rc = ALS_OK;
     if (!k || e->lds <= 0 || e->lds > (int)prop.sharedMemPerBlock) {
         if (e->lds > 65536 && k)
@@ -490,24 +490,24 @@ int als_create(const als_config *cfg, als_engine **out) {
         // tile copy 2 NT KiB: equal at 32 (T + 1) ratings
         e->side[0].restage_max = e->side[1].restage_max = 32 * (e->T + 1);
     }
-    if (const void *k1 = rc ? nullptr : update_kernel_ptr(e->T, e->prec, e->solve, 1)) {
+    if (const void *k1 = rc ? nullptr : update_kernel_ptr(cfg->f, e->prec, e->solve, 1)) {
         if (e->lds > 65536) (void)hipFuncSetAttribute(k1, hipFuncAttributeMaxDynamicSharedMemorySize, e->lds);
         int pc1 = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc1, k1, 64, e->lds) == hipSuccess && pc1 > 0)
             e->grid_v1 = pc1 * e->num_cu;
     }
-    const void *dk = dual_kernel_ptr(e->T, e->prec, e->solve);
+    const void *dk = dual_kernel_ptr(cfg->f, e->prec, e->solve);
     if (!rc && dk) {
-        e->dual_lds = dual_lds_bytes(e->T, e->prec);
+        e->dual_lds = dual_lds_bytes(cfg->f, e->prec);
         int dpc = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&dpc, dk, 64, e->dual_lds) != hipSuccess)
             rc = set_err(e, ALS_E_HIP, "occupancy query failed (dual kernel)");
         e->dual_grid = std::max(1, dpc) * e->num_cu;
-        e->dual_max = dual_max_ratings(e->T, e->prec);
+        e->dual_max = dual_max_ratings(cfg->f, e->prec);
         e->side[0].dual_limit = e->side[1].dual_limit = e->dual_max;
     }
     if (!rc && e->solve == SOLVE_CHOL_REFINE)
-        rc = dev_alloc(e, &e->scratch, (size_t)e->grid_max * (e->T * (e->T + 1) / 2) * 256);
+        rc = dev_alloc(e, &e->scratch, (size_t)e->grid_max * part_floats(cfg->f));
     // Per-dispatch hardware counters (rocprofv3 --pmc) need the two kernels
     // of a half-sweep one after the other: ALS_DUAL_SEQUENTIAL=1 keeps them so.
     if (const char *v = std::getenv("ALS_DUAL_SEQUENTIAL")) e->dual_beside = std::atoi(v) == 0;
@@ -866,7 +866,9 @@ int als_save_libmf(als_engine *e, const char *path) {
 
 namespace {
 
-// Bytes of the saved factorisation of one side: NT tiles of 256 floats per row.
+// Bytes of the saved factorisation of one side: the tiles of the augmented
+// system, 256 floats each, per row (at f = 16T, where the systems are one
+// block smaller, less of it is used).
 int64_t factor_save_bytes(const als_engine *e, int sd) {
     const int64_t rows = sd == 0 ? e->m : e->n;
     return std::max<int64_t>(1, rows) * (int64_t)(e->T * (e->T + 1) / 2) * 256 * (int64_t)sizeof(float);
@@ -904,7 +906,7 @@ int adjoint_impl(als_engine *e, int sd, const float *d_Y, const float *d_X, cons
     a.lambda_bar = d_lambda_bar;
     a.rows = (int)rows;
     a.f = e->cfg.f;
-    if (rows > 0) HIPCHK(e, launch_adjoint_solve(e->T, a, e->stream));
+    if (rows > 0) HIPCHK(e, launch_adjoint_solve(a, e->stream));
     if (d_ybar && cols > 0) {
         if (!e->yb_parts[sd]) {
             // parts of at most YBAR_PART ratings of every column, columns in order
@@ -958,7 +960,7 @@ int adjoint_impl(als_engine *e, int sd, const float *d_Y, const float *d_X, cons
         y.Ybar = d_ybar;
         y.ncols = (int)cols;
         y.f = e->cfg.f;
-        HIPCHK(e, launch_ybar(e->T, y, e->stream));
+        HIPCHK(e, launch_ybar(y, e->stream));
     }
     return ALS_OK;
 }
@@ -1495,7 +1497,7 @@ static int cg_update_x(const float *A, const uint16_t *A16, float *x, const floa
     a.iters = cg_iters;
     a.tol = tol;
     hipStream_t s = reinterpret_cast<hipStream_t>(hip_stream);
-    if (launch_cg_batch((f + 16) / 16, a, s) != hipSuccess) return ALS_E_HIP;
+    if (launch_cg_batch(a, s) != hipSuccess) return ALS_E_HIP;
     if (hipStreamSynchronize(s) != hipSuccess) return ALS_E_HIP;
     return ALS_OK;
 }

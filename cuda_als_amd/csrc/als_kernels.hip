@@ -5,86 +5,106 @@
 
 namespace als {
 
-const void *update_kernel_ptr_p0(int T, int solve, int variant);
-const void *update_kernel_ptr_p1(int T, int solve, int variant);
-const void *update_kernel_ptr_p2(int T, int solve, int variant);
-int update_lds_bytes_p0(int T, int solve, int refine);
-int update_lds_bytes_p1(int T, int solve, int refine);
-int update_lds_bytes_p2(int T, int solve, int refine);
-hipError_t launch_update_p0(int T, int solve, int variant, const UpdateArgs &a, int grid, int lds, hipStream_t s);
-hipError_t launch_update_p1(int T, int solve, int variant, const UpdateArgs &a, int grid, int lds, hipStream_t s);
-hipError_t launch_update_p2(int T, int solve, int variant, const UpdateArgs &a, int grid, int lds, hipStream_t s);
+// _p0, _p1, _p2: FP32, BF16, FP16 Gram; a, b: augmented systems, f = 16T.
+const void *update_kernel_ptr_p0a(int T, int solve, int variant);
+const void *update_kernel_ptr_p0b(int T, int solve, int variant);
+const void *update_kernel_ptr_p1a(int T, int solve, int variant);
+const void *update_kernel_ptr_p1b(int T, int solve, int variant);
+const void *update_kernel_ptr_p2a(int T, int solve, int variant);
+const void *update_kernel_ptr_p2b(int T, int solve, int variant);
+int update_lds_bytes_p0a(int T, int solve);
+int update_lds_bytes_p0b(int T, int solve);
+int update_lds_bytes_p1a(int T, int solve);
+int update_lds_bytes_p1b(int T, int solve);
+int update_lds_bytes_p2a(int T, int solve);
+int update_lds_bytes_p2b(int T, int solve);
+const void *dual_kernel_ptr_p0a(int T, int solve);
+const void *dual_kernel_ptr_p0b(int T, int solve);
+const void *dual_kernel_ptr_p1a(int T, int solve);
+const void *dual_kernel_ptr_p1b(int T, int solve);
+const void *dual_kernel_ptr_p2a(int T, int solve);
+const void *dual_kernel_ptr_p2b(int T, int solve);
+int dual_lds_bytes_p0a(int T);
+int dual_lds_bytes_p0b(int T);
+int dual_lds_bytes_p1a(int T);
+int dual_lds_bytes_p1b(int T);
+int dual_lds_bytes_p2a(int T);
+int dual_lds_bytes_p2b(int T);
+int dual_max_ratings_p0a(int T);
+int dual_max_ratings_p0b(int T);
+int dual_max_ratings_p1a(int T);
+int dual_max_ratings_p1b(int T);
+int dual_max_ratings_p2a(int T);
+int dual_max_ratings_p2b(int T);
 
-const void *update_kernel_ptr(int T, int prec, int solve, int variant) {
+const void *update_kernel_ptr(int f, int prec, int solve, int variant) {
+    const bool aug = augmented(f);
+    const int T = tiles(f);
     switch (prec) {
-    case PREC_FP32: return update_kernel_ptr_p0(T, solve, variant);
-    case PREC_BF16: return update_kernel_ptr_p1(T, solve, variant);
-    case PREC_FP16: return update_kernel_ptr_p2(T, solve, variant);
+    case PREC_FP32: return aug ? update_kernel_ptr_p0a(T, solve, variant) : update_kernel_ptr_p0b(T, solve, variant);
+    case PREC_BF16: return aug ? update_kernel_ptr_p1a(T, solve, variant) : update_kernel_ptr_p1b(T, solve, variant);
+    case PREC_FP16: return aug ? update_kernel_ptr_p2a(T, solve, variant) : update_kernel_ptr_p2b(T, solve, variant);
     default: return nullptr;
     }
 }
 
-int update_lds_bytes(int T, int prec, int solve, int refine) {
+int update_lds_bytes(int f, int prec, int solve) {
+    const bool aug = augmented(f);
+    const int T = tiles(f);
     switch (prec) {
-    case PREC_FP32: return update_lds_bytes_p0(T, solve, refine);
-    case PREC_BF16: return update_lds_bytes_p1(T, solve, refine);
-    case PREC_FP16: return update_lds_bytes_p2(T, solve, refine);
+    case PREC_FP32: return aug ? update_lds_bytes_p0a(T, solve) : update_lds_bytes_p0b(T, solve);
+    case PREC_BF16: return aug ? update_lds_bytes_p1a(T, solve) : update_lds_bytes_p1b(T, solve);
+    case PREC_FP16: return aug ? update_lds_bytes_p2a(T, solve) : update_lds_bytes_p2b(T, solve);
     default: return -1;
     }
 }
 
-hipError_t launch_update(int T, int prec, int solve, int variant, const UpdateArgs &a, int grid, int lds,
-                         hipStream_t s) {
+const void *dual_kernel_ptr(int f, int prec, int solve) {
+    const bool aug = augmented(f);
+    const int T = tiles(f);
     switch (prec) {
-    case PREC_FP32: return launch_update_p0(T, solve, variant, a, grid, lds, s);
-    case PREC_BF16: return launch_update_p1(T, solve, variant, a, grid, lds, s);
-    case PREC_FP16: return launch_update_p2(T, solve, variant, a, grid, lds, s);
-    default: return hipErrorInvalidValue;
-    }
-}
-
-const void *dual_kernel_ptr_p0(int T, int solve);
-const void *dual_kernel_ptr_p1(int T, int solve);
-const void *dual_kernel_ptr_p2(int T, int solve);
-int dual_lds_bytes_p0(int T);
-int dual_lds_bytes_p1(int T);
-int dual_lds_bytes_p2(int T);
-int dual_max_ratings_p0(int T);
-int dual_max_ratings_p1(int T);
-int dual_max_ratings_p2(int T);
-
-const void *dual_kernel_ptr(int T, int prec, int solve) {
-    switch (prec) {
-    case PREC_FP32: return dual_kernel_ptr_p0(T, solve);
-    case PREC_BF16: return dual_kernel_ptr_p1(T, solve);
-    case PREC_FP16: return dual_kernel_ptr_p2(T, solve);
+    case PREC_FP32: return aug ? dual_kernel_ptr_p0a(T, solve) : dual_kernel_ptr_p0b(T, solve);
+    case PREC_BF16: return aug ? dual_kernel_ptr_p1a(T, solve) : dual_kernel_ptr_p1b(T, solve);
+    case PREC_FP16: return aug ? dual_kernel_ptr_p2a(T, solve) : dual_kernel_ptr_p2b(T, solve);
     default: return nullptr;
     }
 }
 
-int dual_lds_bytes(int T, int prec) {
+int dual_lds_bytes(int f, int prec) {
+    const bool aug = augmented(f);
+    const int T = tiles(f);
     switch (prec) {
-    case PREC_FP32: return dual_lds_bytes_p0(T);
-    case PREC_BF16: return dual_lds_bytes_p1(T);
-    case PREC_FP16: return dual_lds_bytes_p2(T);
+    case PREC_FP32: return aug ? dual_lds_bytes_p0a(T) : dual_lds_bytes_p0b(T);
+    case PREC_BF16: return aug ? dual_lds_bytes_p1a(T) : dual_lds_bytes_p1b(T);
+    case PREC_FP16: return aug ? dual_lds_bytes_p2a(T) : dual_lds_bytes_p2b(T);
     default: return 0;
     }
 }
 
-int dual_max_ratings(int T, int prec) {
+int dual_max_ratings(int f, int prec) {
+    const bool aug = augmented(f);
+    const int T = tiles(f);
     switch (prec) {
-    case PREC_FP32: return dual_max_ratings_p0(T);
-    case PREC_BF16: return dual_max_ratings_p1(T);
-    case PREC_FP16: return dual_max_ratings_p2(T);
+    case PREC_FP32: return aug ? dual_max_ratings_p0a(T) : dual_max_ratings_p0b(T);
+    case PREC_BF16: return aug ? dual_max_ratings_p1a(T) : dual_max_ratings_p1b(T);
+    case PREC_FP16: return aug ? dual_max_ratings_p2a(T) : dual_max_ratings_p2b(T);
     default: return 0;
     }
 }
 
-hipError_t launch_dual(int T, int prec, int solve, const UpdateArgs &a, int grid, int lds, hipStream_t s) {
-    const void *k = dual_kernel_ptr(T, prec, solve);
+static hipError_t launch_rows(const void *k, const UpdateArgs &a, int grid, int lds, hipStream_t s) {
     if (!k) return hipErrorInvalidValue;
     void *args[] = {const_cast<UpdateArgs *>(&a)};
     return hipLaunchKernel(k, dim3(grid), dim3(WAVE), args, (size_t)lds, s);
+}
+
+hipError_t launch_update(int f, int prec, int solve, int variant, const UpdateArgs &a, int grid, int lds,
+                         hipStream_t s) {
+    return launch_rows(update_kernel_ptr(f, prec, solve, variant), a, grid, lds, s);
+}
+
+hipError_t launch_dual(int f, int prec, int solve, const UpdateArgs &a, int grid, int lds, hipStream_t s) {
+    return launch_rows(dual_kernel_ptr(f, prec, solve), a, grid, lds, s);
 }
 
 // ------------------------------------------------------------------ RMSE
@@ -198,13 +218,13 @@ hipError_t launch_to16(int prec, const float *src, uint16_t *dst, int64_t count,
 // g_u = dL/dx_u, with the Cholesky factor saved by the forward pass:
 //   xbar_u = A_u^-1 g_u  (forward + back substitution on the saved factor)
 //   dL/dlambda_u = -n_u xbar_u . x_u
-template <int T>
+template <int T, bool AUG>
 __global__ __launch_bounds__(WAVE) void adjoint_solve_kernel(AdjointArgs a) {
-    constexpr int FP = 16 * T, NT = T * (T + 1) / 2;
+    constexpr int LD = AUG ? 16 * T : 16 * T + 16, NT = T * (T + 1) / 2;
     const int l = lane(), f = a.f;
     for (int row = blockIdx.x; row < a.rows; row += gridDim.x) {
         const int n = a.ptr[row + 1] - a.ptr[row];
-        const int64_t o = (int64_t)row * FP;
+        const int64_t o = (int64_t)row * LD;
         float g[T];
 #pragma unroll
         for (int J = 0; J < T; ++J) g[J] = 0.f;
@@ -222,7 +242,7 @@ __global__ __launch_bounds__(WAVE) void adjoint_solve_kernel(AdjointArgs a) {
             load_colform<T>(a.X + o, f, x);
             lb = -(float)n * colform_dot(g, x, T);
         }
-        store_colform<T>(a.Xbar + o, g);
+        store_colform<T, !AUG>(a.Xbar + o, g);
         if (l == 0) a.lambda_bar[row] = lb;
     }
 }
@@ -235,13 +255,13 @@ __global__ __launch_bounds__(WAVE) void adjoint_solve_kernel(AdjointArgs a) {
 // c + 16(T-1); the two dots are 16-lane sums; the groups' sums are added at
 // the end and written as the part's row. ybar_sum_kernel: one wave per
 // column adds its parts' rows in part order.
-template <int T>
+template <int T, bool AUG>
 __global__ __launch_bounds__(WAVE) void ybar_part_kernel(YbarArgs a) {
-    constexpr int FP = 16 * T;
+    constexpr int FP = 16 * T, LD = AUG ? FP : FP + 16;
     const int l = lane(), c = l & 15, grp = l >> 4, f = a.f;
     for (int p = blockIdx.x; p < a.nparts; p += gridDim.x) {
         const int4 pt = a.parts[p];
-        const int64_t oy = (int64_t)pt.x * FP;
+        const int64_t oy = (int64_t)pt.x * LD;
         float y[T], ac[T];
 #pragma unroll
         for (int J = 0; J < T; ++J) {
@@ -250,7 +270,7 @@ __global__ __launch_bounds__(WAVE) void ybar_part_kernel(YbarArgs a) {
             ac[J] = 0.f;
         }
         for (int k = pt.y + grp; k < pt.z; k += 4) {
-            const int64_t ox = (int64_t)a.cidx[k] * FP;
+            const int64_t ox = (int64_t)a.cidx[k] * LD;
             const float r = a.cval[k];
             float x[T], b[T], pxy = 0.f, pby = 0.f;
 #pragma unroll
@@ -281,9 +301,9 @@ __global__ __launch_bounds__(WAVE) void ybar_part_kernel(YbarArgs a) {
     }
 }
 
-template <int T>
+template <int T, bool AUG>
 __global__ __launch_bounds__(WAVE) void ybar_sum_kernel(YbarArgs a) {
-    constexpr int FP = 16 * T, NJ = (FP + WAVE - 1) / WAVE;
+    constexpr int FP = 16 * T, LD = AUG ? FP : FP + 16, NJ = (LD + WAVE - 1) / WAVE;
     const int l = lane(), f = a.f;
     for (int col = blockIdx.x; col < a.ncols; col += gridDim.x) {
         float s[NJ];
@@ -299,7 +319,7 @@ __global__ __launch_bounds__(WAVE) void ybar_sum_kernel(YbarArgs a) {
 #pragma unroll
         for (int m = 0; m < NJ; ++m) {
             const int j = WAVE * m + l;
-            if (j < FP) a.Ybar[(int64_t)col * FP + j] = j < f ? s[m] : 0.f;
+            if (j < LD) a.Ybar[(int64_t)col * LD + j] = j < f ? s[m] : 0.f;
         }
     }
 }
@@ -402,9 +422,9 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(T <= 7 ? 2
     }
 }
 
-hipError_t launch_cg_batch(int T, const CgBatchArgs &a, hipStream_t s) {
+hipError_t launch_cg_batch(const CgBatchArgs &a, hipStream_t s) {
     const int grid = std::max(1, std::min(a.batch, 65536));
-    switch (T) {
+    switch (tiles(a.f)) {
 #define ALS_CGB(TT) case TT: cg_batch_kernel<TT><<<grid, WAVE, 0, s>>>(a); break;
     ALS_CGB(1) ALS_CGB(2) ALS_CGB(3) ALS_CGB(4) ALS_CGB(5) ALS_CGB(6) ALS_CGB(7) ALS_CGB(8) ALS_CGB(9)
 #undef ALS_CGB
@@ -413,31 +433,36 @@ hipError_t launch_cg_batch(int T, const CgBatchArgs &a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_adjoint_solve(int T, const AdjointArgs &a, hipStream_t s) {
-    const int grid = std::max(1, std::min(a.rows, 65536));
-    const size_t lds = 0;
-    switch (T) {
-#define ALS_ADJ(TT) case TT: adjoint_solve_kernel<TT><<<grid, WAVE, lds, s>>>(a); break;
-    ALS_ADJ(1) ALS_ADJ(2) ALS_ADJ(3) ALS_ADJ(4) ALS_ADJ(5) ALS_ADJ(6) ALS_ADJ(7) ALS_ADJ(8) ALS_ADJ(9)
-#undef ALS_ADJ
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+template <int T, bool AUG>
+static void adjoint_solve(const AdjointArgs &a, hipStream_t s) {
+    adjoint_solve_kernel<T, AUG><<<std::max(1, std::min(a.rows, 65536)), WAVE, 0, s>>>(a);
 }
 
-hipError_t launch_ybar(int T, const YbarArgs &a, hipStream_t s) {
-    const int gp = std::max(1, std::min(a.nparts, 65536)), gc = std::max(1, std::min(a.ncols, 65536));
-    switch (T) {
-#define ALS_YB(TT)                                                   \
-    case TT:                                                         \
-        ybar_part_kernel<TT><<<gp, WAVE, 0, s>>>(a);                 \
-        ybar_sum_kernel<TT><<<gc, WAVE, 0, s>>>(a);                  \
-        break;
-    ALS_YB(1) ALS_YB(2) ALS_YB(3) ALS_YB(4) ALS_YB(5) ALS_YB(6) ALS_YB(7) ALS_YB(8) ALS_YB(9)
-#undef ALS_YB
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+template <int T, bool AUG>
+static void ybar(const YbarArgs &a, hipStream_t s) {
+    ybar_part_kernel<T, AUG><<<std::max(1, std::min(a.nparts, 65536)), WAVE, 0, s>>>(a);
+    ybar_sum_kernel<T, AUG><<<std::max(1, std::min(a.ncols, 65536)), WAVE, 0, s>>>(a);
 }
+
+// FN<T, AUG> for a's f; f = 16T needs no ninth block (f <= 143).
+#define ALS_BY_TILES(FN)                                                        \
+    switch (tiles(a.f)) {                                                       \
+    case 1: augmented(a.f) ? FN<1, true>(a, s) : FN<1, false>(a, s); break;     \
+    case 2: augmented(a.f) ? FN<2, true>(a, s) : FN<2, false>(a, s); break;     \
+    case 3: augmented(a.f) ? FN<3, true>(a, s) : FN<3, false>(a, s); break;     \
+    case 4: augmented(a.f) ? FN<4, true>(a, s) : FN<4, false>(a, s); break;     \
+    case 5: augmented(a.f) ? FN<5, true>(a, s) : FN<5, false>(a, s); break;     \
+    case 6: augmented(a.f) ? FN<6, true>(a, s) : FN<6, false>(a, s); break;     \
+    case 7: augmented(a.f) ? FN<7, true>(a, s) : FN<7, false>(a, s); break;     \
+    case 8: augmented(a.f) ? FN<8, true>(a, s) : FN<8, false>(a, s); break;     \
+    case 9: FN<9, true>(a, s); break;                                           \
+    default: return hipErrorInvalidValue;                                       \
+    }                                                                           \
+    return hipGetLastError();
+
+hipError_t launch_adjoint_solve(const AdjointArgs &a, hipStream_t s) { ALS_BY_TILES(adjoint_solve) }
+
+hipError_t launch_ybar(const YbarArgs &a, hipStream_t s) { ALS_BY_TILES(ybar) }
+#undef ALS_BY_TILES
 
 }  // namespace als

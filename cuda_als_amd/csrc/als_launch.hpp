@@ -12,13 +12,32 @@ enum Prec { PREC_FP32 = 0, PREC_BF16 = 1, PREC_FP16 = 2 };
 enum SolveKind { SOLVE_CHOL = 0, SOLVE_CG = 1, SOLVE_CHOL_REFINE = 2, SOLVE_CHOL_WARM = 3 };
 constexpr int MAX_T = 9;  // augmented dimension f + 1 <= 16 * MAX_T
 
+// The system a row solves is held in T x T blocks of 16. b = sum r y rides
+// along as row f of an augmented matrix where the last block has room for it
+// (f % 16 != 0); where f is a multiple of 16 that row would take a block of
+// its own (T + 1 more 16x16 tiles: 15 instead of 10 at f = 64, 45 instead of
+// 36 at f = 128), and b is summed beside the tiles instead. One sweep at the
+// ml10M shape (69,878 x 10,677, 9.0M ratings), row in the tiles -> beside:
+// f = 80 FP16 Gram and CG 0.80 -> 0.70 ms, f = 64 FP32 1.71 -> 1.50 ms, three
+// warm-started BF16 models of f = 32, 64, 128 together 3.25 -> 2.79 ms.
+constexpr int tiles(int f) { return (f + 15) / 16; }
+constexpr bool augmented(int f) { return f % 16 != 0; }
+// Row stride (floats, or halves of the 16-bit shadow) of every factor matrix:
+// the augmented system's, whatever the solve uses.
+constexpr int row_stride(int f) { return 16 * ((f + 16) / 16); }
+// Floats of one part of a split row or of one copy of a system: its tiles,
+// and b where it is not in them.
+constexpr int part_floats(int f) { return tiles(f) * (tiles(f) + 1) / 2 * 256 + (augmented(f) ? 0 : f); }
+// Floats of one row's saved factor.
+constexpr int factor_floats(int f) { return tiles(f) * (tiles(f) + 1) / 2 * 256; }
+
 struct UpdateArgs {
     const int *ptr;             // CSR of the side being updated (int32, reference layout)
     const int *idx;
     const float *val;
-    const float *Y;             // fixed factors, FP32, row stride 16*T
-    const uint16_t *Ys;         // fixed factors, 16-bit shadow, row stride 16*T (16-bit Gram only)
-    float *X;                   // updated factors, FP32, row stride 16*T (CG: warm start in)
+    const float *Y;             // fixed factors, FP32, row stride row_stride(f)
+    const uint16_t *Ys;         // fixed factors, 16-bit shadow, the same stride (16-bit Gram only)
+    float *X;                   // updated factors, FP32, the same stride (CG: warm start in)
     uint16_t *Xs;               // 16-bit shadow of X to refresh (nullable)
     const float *lambda_rows;   // per-row lambda (nullable -> lambda)
     float lambda;
@@ -26,7 +45,7 @@ struct UpdateArgs {
     const int4 *units;          // {row, kb, ke, split} work units, heaviest first
     const int4 *splits;         // {slot_base, nparts, part_len, -} per split row
     int *counters;              // arrivals per split row (0 between launches)
-    float *partial;             // partial Gram tiles, NT*256 floats per slot
+    float *partial;             // partial Gram tiles (and b), part_floats(f) per slot
     const int *batch_begin;     // batch b = units[batch_begin[b] .. batch_begin[b+1])
     int nbatches;
     int *queue;                 // next ticket (0 between launches)
@@ -38,9 +57,9 @@ struct UpdateArgs {
     int restage_max;            // whole rows up to this many ratings form the residual by
                                 // restaging their ratings; longer ones use the tile copy
     int *fail_count;            // rows whose solve broke down (x set to 0)
-    float *Lsave;               // Cholesky factor tiles per row, NT*256 floats (nullable)
-    float *scratch;             // per-wave copy of A for refinement, NT*256 floats per workgroup
-    const float *zero32;        // one row of zeros (16*T floats) read by unused chunk slots
+    float *Lsave;               // Cholesky factor tiles per row, factor_floats(f) (nullable)
+    float *scratch;             // per-wave copy of A (and b) for refinement, part_floats(f) per workgroup
+    const float *zero32;        // one row of zeros (row_stride(f) floats) read by unused chunk slots
     const uint16_t *zero16;     // same, 16-bit
     int ys_bytes;               // bytes of the 16-bit Y shadow when below 2^31 (the pipelined
                                 // Gram then gathers with 32-bit buffer offsets), else 0
@@ -48,9 +67,9 @@ struct UpdateArgs {
                                 // (gram_dma_built), 0: through registers
 };
 
-// Tile counts and precisions whose update kernels carry the LDS-DMA Gram:
-// a 16-bit Gram, at most 8 tiles (a chunk's gather tasks fit a wave) and
-// T % 4 != 0 (rows of 16T halves keep a transposing read on distinct banks).
+// Augmented tile counts (als_info.T) and precisions whose update kernels carry
+// the LDS-DMA Gram: a 16-bit Gram, at most 8 tiles (a chunk's gather tasks fit
+// a wave) and T % 4 != 0.
 constexpr bool gram_dma_built(int T, int prec) { return prec != PREC_FP32 && T <= 8 && T % 4 != 0; }
 
 // Several models (different f) on one rating matrix, one launch: batch b of
@@ -59,10 +78,10 @@ constexpr int MAX_MODELS = 4;  // engines per group (als_group_*)
 
 struct AdjointArgs {
     const int *ptr;             // CSR of the side that was updated
-    const float *X;             // forward solution, stride 16*T
+    const float *X;             // forward solution, stride row_stride(f)
     const float *Lsave;         // packed factors from the forward pass
-    const float *Gbar;          // dL/dX, stride 16*T
-    float *Xbar;                // A^-1 Gbar, stride 16*T
+    const float *Gbar;          // dL/dX, the same stride
+    float *Xbar;                // A^-1 Gbar, the same stride
     float *lambda_bar;          // -n_u Xbar_u . X_u
     int rows;
     int f;
@@ -89,8 +108,8 @@ struct YbarArgs {
     const int *cptr;            // CSC of the same matrix (columns = fixed-factor rows)
     const int *cidx;
     const float *cval;
-    const float *X, *Xbar, *Y;  // stride 16*T
-    float *Ybar;                // stride 16*T (overwritten)
+    const float *X, *Xbar, *Y;  // stride row_stride(f)
+    float *Ybar;                // the same stride (overwritten)
     int ncols;
     int f;
     // the columns' rating lists cut into parts of at most YBAR_PART ratings:
@@ -98,7 +117,7 @@ struct YbarArgs {
     // colpart[c] .. colpart[c+1]-1, in order; partial: one row per part
     const int4 *parts;
     const int *colpart;
-    float *partial;             // nparts x 16*T
+    float *partial;             // nparts x row_stride(f)
     int nparts;
 };
 constexpr int YBAR_PART = 1024;
@@ -113,23 +132,23 @@ struct RmseArgs {
 };
 
 // Launchers (als_kernels_*.hip). Each returns the hipError_t of the launch.
-int update_lds_bytes(int T, int prec, int solve, int refine);
+int update_lds_bytes(int f, int prec, int solve);
 // variant 0: the default kernel of the solver (two waves per SIMD for the
 // refinement solvers); variant 1: one wave per SIMD (warm-started refinement,
-// T >= 7; null elsewhere).
-hipError_t launch_update(int T, int prec, int solve, int variant, const UpdateArgs &a, int grid, int lds_bytes,
+// f >= 96; null elsewhere).
+hipError_t launch_update(int f, int prec, int solve, int variant, const UpdateArgs &a, int grid, int lds_bytes,
                          hipStream_t s);
-const void *update_kernel_ptr(int T, int prec, int solve, int variant = 0);
+const void *update_kernel_ptr(int f, int prec, int solve, int variant = 0);
 // Light rows through the dual system, one launch per half-sweep after the
 // update kernel (null / 0 where the variant has no dual system: f < 64, CG,
 // classic refinement). dual_max_ratings: rows below it take the dual system.
-const void *dual_kernel_ptr(int T, int prec, int solve);
-int dual_lds_bytes(int T, int prec);
-int dual_max_ratings(int T, int prec);
-hipError_t launch_dual(int T, int prec, int solve, const UpdateArgs &a, int grid, int lds_bytes, hipStream_t s);
-hipError_t launch_adjoint_solve(int T, const AdjointArgs &a, hipStream_t s);
-hipError_t launch_cg_batch(int T, const CgBatchArgs &a, hipStream_t s);
-hipError_t launch_ybar(int T, const YbarArgs &a, hipStream_t s);
+const void *dual_kernel_ptr(int f, int prec, int solve);
+int dual_lds_bytes(int f, int prec);
+int dual_max_ratings(int f, int prec);
+hipError_t launch_dual(int f, int prec, int solve, const UpdateArgs &a, int grid, int lds_bytes, hipStream_t s);
+hipError_t launch_adjoint_solve(const AdjointArgs &a, hipStream_t s);
+hipError_t launch_cg_batch(const CgBatchArgs &a, hipStream_t s);
+hipError_t launch_ybar(const YbarArgs &a, hipStream_t s);
 // RMSE partial sums of a.n ratings over `blocks` blocks into a.partials
 // (blocks doubles), then out[0] = their sum (with_rmse: out[1] = sqrt(sum / n)).
 constexpr int RMSE_BLOCKS = 1024;

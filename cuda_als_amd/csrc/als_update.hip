@@ -1,151 +1,99 @@
 // Instantiates the per-row update kernel for one Gram precision (ALS_PREC is
-// set by the build: 0 FP32, 1 BF16, 2 FP16), all tile counts T = 1..9 and
-// both solvers. Compiled once per precision so the three build in parallel.
+// set by the build: 0 FP32, 1 BF16, 2 FP16) and one form of the system
+// (ALS_AUG: 1 augmented, T = 1..9; 0 f = 16T, T = 1..8), every solver.
+// Compiled once per pair so that they build in parallel.
 #include "als_device.hpp"
 
 #ifndef ALS_PREC
 #error "ALS_PREC must be defined"
 #endif
+#ifndef ALS_AUG
+#error "ALS_AUG must be defined"
+#endif
 
 namespace als {
 
-template <int S>
-static const void *kernel_w2_for(int T) {
-    switch (T) {
-    case 1: return (const void *)&update_kernel_w2<1, ALS_PREC, S>;
-    case 2: return (const void *)&update_kernel_w2<2, ALS_PREC, S>;
-    case 3: return (const void *)&update_kernel_w2<3, ALS_PREC, S>;
-    case 4: return (const void *)&update_kernel_w2<4, ALS_PREC, S>;
-    case 5: return (const void *)&update_kernel_w2<5, ALS_PREC, S>;
-    case 6: return (const void *)&update_kernel_w2<6, ALS_PREC, S>;
-    case 7: return (const void *)&update_kernel_w2<7, ALS_PREC, S>;
-    case 8: return (const void *)&update_kernel_w2<8, ALS_PREC, S>;
-    case 9: return (const void *)&update_kernel_w2<9, ALS_PREC, S>;
-    default: return nullptr;
-    }
+constexpr bool AUG = ALS_AUG != 0;
+constexpr int LAST_T = AUG ? MAX_T : MAX_T - 1;
+template <int T> using Sys = Geo<T, ALS_PREC, AUG>;
+
+// FN<T>(args) for a tile count known at run time, T in FIRST .. LAST_T; BAD
+// outside.
+template <int FIRST, class FN, class R>
+static R by_tiles(int T, FN fn, R bad) {
+    if constexpr (FIRST > LAST_T) return bad;
+    else return T == FIRST ? fn(std::integral_constant<int, FIRST>{}) : by_tiles<FIRST + 1>(T, fn, bad);
 }
 
-// One wave per SIMD (no waves-per-EU bound: the whole register file for one
-// wave, spill-free at the widest tile counts); selectable per side.
-template <int S>
-static const void *kernel_w1_for(int T) {
-    switch (T) {
-    case 7: return (const void *)&update_kernel<7, ALS_PREC, S>;
-    case 8: return (const void *)&update_kernel<8, ALS_PREC, S>;
-    case 9: return (const void *)&update_kernel<9, ALS_PREC, S>;
-    default: return nullptr;
-    }
+// S at T tiles. Variant 1: one wave per SIMD (no waves-per-EU bound: the
+// whole register file for one wave, spill-free at the widest tile counts),
+// built for the warm-started solver at f >= 96; selectable per side.
+static const void *update_kernel_for(int T, int solve, int variant) {
+    return by_tiles<1>(
+        T,
+        [&](auto t) -> const void * {
+            constexpr int N = decltype(t)::value;
+            if (variant == 1) {
+                if constexpr (Sys<N>::TA >= 7)
+                    return solve == SOLVE_CHOL_WARM ? (const void *)&update_kernel<N, ALS_PREC, SOLVE_CHOL_WARM, AUG>
+                                                    : nullptr;
+                return nullptr;
+            }
+            if (variant != 0) return nullptr;
+            return solve == SOLVE_CHOL  ? (const void *)&update_kernel<N, ALS_PREC, SOLVE_CHOL, AUG>
+                   : solve == SOLVE_CG  ? (const void *)&update_kernel<N, ALS_PREC, SOLVE_CG, AUG>
+                   : solve == SOLVE_CHOL_WARM
+                       ? (const void *)&update_kernel_w2<N, ALS_PREC, SOLVE_CHOL_WARM, AUG>
+                       : (const void *)&update_kernel_w2<N, ALS_PREC, SOLVE_CHOL_REFINE, AUG>;
+        },
+        (const void *)nullptr);
 }
 
-template <int S>
-static const void *kernel_for(int T) {
-    switch (T) {
-    case 1: return (const void *)&update_kernel<1, ALS_PREC, S>;
-    case 2: return (const void *)&update_kernel<2, ALS_PREC, S>;
-    case 3: return (const void *)&update_kernel<3, ALS_PREC, S>;
-    case 4: return (const void *)&update_kernel<4, ALS_PREC, S>;
-    case 5: return (const void *)&update_kernel<5, ALS_PREC, S>;
-    case 6: return (const void *)&update_kernel<6, ALS_PREC, S>;
-    case 7: return (const void *)&update_kernel<7, ALS_PREC, S>;
-    case 8: return (const void *)&update_kernel<8, ALS_PREC, S>;
-    case 9: return (const void *)&update_kernel<9, ALS_PREC, S>;
-    default: return nullptr;
-    }
-}
-
-template <int T>
-static int lds_for(int solve, int refine) {
-    (void)refine;
-    return solve == SOLVE_CHOL_REFINE ? Geo<T, ALS_PREC>::refine_lds_bytes() : Geo<T, ALS_PREC>::lds_bytes();
-}
-
-#define ALS_CAT2(a, b) a##b
-#define ALS_CAT(a, b) ALS_CAT2(a, b)
-
-const void *ALS_CAT(update_kernel_ptr_p, ALS_PREC)(int T, int solve, int variant) {
-    if (variant == 1) return solve == SOLVE_CHOL_WARM ? kernel_w1_for<SOLVE_CHOL_WARM>(T) : nullptr;
-    if (variant != 0) return nullptr;
-    return solve == SOLVE_CHOL        ? kernel_for<SOLVE_CHOL>(T)
-           : solve == SOLVE_CG        ? kernel_for<SOLVE_CG>(T)
-           : solve == SOLVE_CHOL_WARM ? kernel_w2_for<SOLVE_CHOL_WARM>(T)
-                                      : kernel_w2_for<SOLVE_CHOL_REFINE>(T);
-}
-
-int ALS_CAT(update_lds_bytes_p, ALS_PREC)(int T, int solve, int refine) {
-    switch (T) {
-    case 1: return lds_for<1>(solve, refine);
-    case 2: return lds_for<2>(solve, refine);
-    case 3: return lds_for<3>(solve, refine);
-    case 4: return lds_for<4>(solve, refine);
-    case 5: return lds_for<5>(solve, refine);
-    case 6: return lds_for<6>(solve, refine);
-    case 7: return lds_for<7>(solve, refine);
-    case 8: return lds_for<8>(solve, refine);
-    case 9: return lds_for<9>(solve, refine);
-    default: return -1;
-    }
-}
-
-template <int T, int S>
-static const void *dual_one() {
-    if constexpr (Geo<T, ALS_PREC>::DUAL_TD > 0) return (const void *)&dual_kernel<T, ALS_PREC, S>;
-    else return nullptr;
-}
-
-template <int S>
-static const void *dual_for(int T) {
-    switch (T) {
-    case 5: return dual_one<5, S>();
-    case 6: return dual_one<6, S>();
-    case 7: return dual_one<7, S>();
-    case 8: return dual_one<8, S>();
-    case 9: return dual_one<9, S>();
-    default: return nullptr;
-    }
-}
-
-// The dual system exists for T >= 5 (Geo::DUAL_TD > 0), after the plain
+// The dual system exists for f >= 64 (Geo::DUAL_TD > 0), after the plain
 // Cholesky solve or the warm-started one.
-const void *ALS_CAT(dual_kernel_ptr_p, ALS_PREC)(int T, int solve) {
-    return solve == SOLVE_CHOL        ? dual_for<SOLVE_CHOL>(T)
-           : solve == SOLVE_CHOL_WARM ? dual_for<SOLVE_CHOL_WARM>(T)
-                                      : nullptr;
+static const void *dual_kernel_for(int T, int solve) {
+    return by_tiles<1>(
+        T,
+        [&](auto t) -> const void * {
+            constexpr int N = decltype(t)::value;
+            if constexpr (Sys<N>::DUAL_TD > 0)
+                return solve == SOLVE_CHOL        ? (const void *)&dual_kernel<N, ALS_PREC, SOLVE_CHOL, AUG>
+                       : solve == SOLVE_CHOL_WARM ? (const void *)&dual_kernel<N, ALS_PREC, SOLVE_CHOL_WARM, AUG>
+                                                  : nullptr;
+            return nullptr;
+        },
+        (const void *)nullptr);
 }
 
-template <int T>
-static int dual_lds_for() {
-    using G = Geo<T, ALS_PREC>;
-    return G::dual_lds_bytes();
+#define ALS_CAT2(a, b, c) a##b##c
+#define ALS_CAT(a, b, c) ALS_CAT2(a, b, c)
+#if ALS_AUG
+#define ALS_NAME(x) ALS_CAT(x##_p, ALS_PREC, a)
+#else
+#define ALS_NAME(x) ALS_CAT(x##_p, ALS_PREC, b)
+#endif
+
+const void *ALS_NAME(update_kernel_ptr)(int T, int solve, int variant) { return update_kernel_for(T, solve, variant); }
+
+int ALS_NAME(update_lds_bytes)(int T, int solve) {
+    return by_tiles<1>(
+        T,
+        [&](auto t) {
+            using G = Sys<decltype(t)::value>;
+            return solve == SOLVE_CHOL_REFINE ? G::refine_lds_bytes() : G::lds_bytes();
+        },
+        -1);
 }
 
-int ALS_CAT(dual_lds_bytes_p, ALS_PREC)(int T) {
-    switch (T) {
-    case 5: return dual_lds_for<5>();
-    case 6: return dual_lds_for<6>();
-    case 7: return dual_lds_for<7>();
-    case 8: return dual_lds_for<8>();
-    case 9: return dual_lds_for<9>();
-    default: return 0;
-    }
+const void *ALS_NAME(dual_kernel_ptr)(int T, int solve) { return dual_kernel_for(T, solve); }
+
+int ALS_NAME(dual_lds_bytes)(int T) {
+    return by_tiles<1>(
+        T, [](auto t) { return Sys<decltype(t)::value>::DUAL_TD > 0 ? Sys<decltype(t)::value>::dual_lds_bytes() : 0; }, 0);
 }
 
-int ALS_CAT(dual_max_ratings_p, ALS_PREC)(int T) {
-    switch (T) {
-    case 5: return 16 * Geo<5, ALS_PREC>::DUAL_TD;
-    case 6: return 16 * Geo<6, ALS_PREC>::DUAL_TD;
-    case 7: return 16 * Geo<7, ALS_PREC>::DUAL_TD;
-    case 8: return 16 * Geo<8, ALS_PREC>::DUAL_TD;
-    case 9: return 16 * Geo<9, ALS_PREC>::DUAL_TD;
-    default: return 0;
-    }
-}
-
-hipError_t ALS_CAT(launch_update_p, ALS_PREC)(int T, int solve, int variant, const UpdateArgs &a, int grid, int lds,
-                                             hipStream_t s) {
-    const void *k = ALS_CAT(update_kernel_ptr_p, ALS_PREC)(T, solve, variant);
-    if (!k) return hipErrorInvalidValue;
-    void *args[] = {const_cast<UpdateArgs *>(&a)};
-    return hipLaunchKernel(k, dim3(grid), dim3(WAVE), args, (size_t)lds, s);
+int ALS_NAME(dual_max_ratings)(int T) {
+    return by_tiles<1>(T, [](auto t) { return 16 * Sys<decltype(t)::value>::DUAL_TD; }, 0);
 }
 
 }  // namespace als

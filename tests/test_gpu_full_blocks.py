@@ -1,0 +1,94 @@
+"""Ranks that fill their 16-column blocks (f = 16T): the systems are kept in T
+blocks with the right-hand side beside them instead of an augmented row in a
+block of its own. Every such rank, Gram precision and solver against the FP64
+oracle, on rows that end at every place of a 32-rating chunk, whole and split
+(so that b travels with the parts), and the neighbouring ranks 16T - 1 and
+16T + 1 that keep the augmented form."""
+import numpy as np
+import pytest
+
+import cuda_als_amd as ca
+from cuda_als_amd import engine as E
+from oracle import als_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [0, 1, 2, 15, 16, 17, 31, 32, 33, 47, 48, 63, 64, 65, 79, 80, 81, 96, 97, 128, 150, 193, 256, 300]
+COLS = 320
+ORACLE_PREC = {E.Prec.FP32: O.PREC_EXACT, E.Prec.BF16: O.PREC_BF16, E.Prec.FP16: O.PREC_FP16}
+
+
+def matrix(f):
+    rng = np.random.default_rng(f)
+    idx = np.concatenate([np.sort(rng.choice(COLS, n, replace=False)) for n in LENGTHS]).astype(np.int32)
+    val = rng.integers(1, 11, idx.size) / 2.0
+    ptr = np.concatenate([[0], np.cumsum(LENGTHS)])
+    d = ca.from_arrays(len(LENGTHS), COLS, ptr, idx, val, [0], [0], [3.0])
+    return d, (0.4 * rng.standard_normal((len(LENGTHS), f))).astype(np.float32), \
+        (0.4 * rng.standard_normal((COLS, f))).astype(np.float32)
+
+
+def rel(got, want):
+    return (np.abs(got - want).max(axis=1) / np.maximum(1.0, np.abs(want).max(axis=1))).max()
+
+
+# (solver, refinement steps, warm): against the oracle on the Gram's own rounded inputs, but for the classic
+# refinement, whose residual is restaged from the FP32 rows and which converges to the exact system's solution
+SOLVES = {"chol": (E.SolveType.CHOL, 0, False), "warm": (E.SolveType.CHOL, 1, True),
+          "refined": (E.SolveType.CHOL, 2, False), "cg": (E.SolveType.CUMF_ALS_CG_FP32, 0, False)}
+
+
+# parts of split rows refine against the 16-bit system, so the refined solver runs unsplit
+@pytest.mark.parametrize("solve,split_len", [(s, n) for s in SOLVES for n in (0, 40) if (s, n) != ("refined", 40)])
+@pytest.mark.parametrize("prec", list(ORACLE_PREC))
+@pytest.mark.parametrize("f", [15, 16, 17, 32, 48, 63, 64, 65, 80, 96, 112, 127, 128, 129])
+def test_half_sweep(f, prec, solve, split_len):
+    """Within 1e-4 of the FP64 oracle, as the other half-sweep tests ask (the
+    oracle's system is formed from the same rounded factors, so the precision
+    of the Gram's inputs is not in the difference; the FP32 solve of these
+    rows is a few 1e-6 off, the refined one of BF16 rows, whose two steps
+    each gain about two digits, a few 1e-5)."""
+    d, U0, V0 = matrix(f)
+    kind, refine, warm = SOLVES[solve]
+    oprec = O.PREC_EXACT if solve == "refined" else ORACLE_PREC[prec]
+    cfg = O.config(f, 0.05, O.SOLVE_CG if solve == "cg" else O.SOLVE_CHOL, cg_tol=0.0, gram_prec=oprec)
+    want = O.update_rows(cfg, np.arange(d.m), d.csr_ptr, d.csr_idx, d.csr_val, V0.astype(np.float64),
+                         U0.astype(np.float64) if solve == "cg" else None)
+    with E.Engine(E.make_config(f, 0.05, 1, kind, prec, refine=refine, refine_warm=warm, cg_tol=0.0,
+                                split_len=split_len), d) as e:
+        if solve == "refined":
+            e.set_schedule(ca.ALS_SIDE_USERS, 0, 0, 1 << 30)
+        e.set_factors(ca.ALS_SIDE_USERS, U0)
+        e.set_factors(ca.ALS_SIDE_ITEMS, V0)
+        e.update(ca.ALS_SIDE_USERS)
+        got = e.get_factors(ca.ALS_SIDE_USERS)
+        info = e.info()
+        assert info.failures == 0 and (info.nsplit_rows[0] > 0) == (split_len > 0)
+    print(f, prec, solve, split_len, rel(got, want))
+    assert not got[0].any() and rel(got, want) <= 1e-4
+
+
+@pytest.mark.parametrize("prec", [E.Prec.FP32, E.Prec.FP16])
+@pytest.mark.parametrize("f", [16, 64, 128])
+def test_padding_of_caller_buffers(f, prec):
+    """als_forward_dev writes whole rows of the caller's X, zeros past column
+    f, whatever was there, and the adjoint does the same for its outputs."""
+    import torch
+    d, _, V0 = matrix(f)
+    with E.Engine(E.make_config(f, 0.05, 1, E.SolveType.CHOL, prec), d) as e:
+        ld = e.info().ld
+        s = torch.cuda.Stream()
+        e.set_stream(s.cuda_stream)
+        Y = torch.zeros(d.n, ld, device="cuda")
+        Y[:, :f] = torch.tensor(V0, device="cuda")
+        X, xbar, ybar = (torch.full((r, ld), 7.0, device="cuda") for r in (d.m, d.m, d.n))
+        g = torch.zeros(d.m, ld, device="cuda")
+        g[:, :f] = 1e-2
+        lbar = torch.zeros(d.m, device="cuda")
+        torch.cuda.synchronize()
+        e.forward_dev(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), None)
+        e.adjoint_dev(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), g.data_ptr(), xbar.data_ptr(), lbar.data_ptr(),
+                      ybar.data_ptr())
+        torch.cuda.synchronize()
+        for t in (X, xbar, ybar):
+            assert not t[:, f:].any() and t[:, :f].any()
