@@ -9,7 +9,8 @@
 //      time, into LDS, with the rating r_i written into the spare column f
 //      ("augmented" row [y_i | r_i]).
 //   2. Accumulate the lower-triangle 16x16 tiles of G = sum [y r]^T [y r] on
-//      MFMA (FP32 16x16x4, or BF16/FP16 16x16x32 with FP32 accumulators).
+//      MFMA (BF16/FP16 16x16x32 with FP32 accumulators; FP32 values as sums
+//      of three BF16 parts).
 //      G[0:f,0:f] is the Gram sum y y^T (reference als_model.cu:91-167),
 //      G[f,0:f] is b = sum r y (reference RHS, als_model.cu:1816-1852).
 //   3. Add lambda * n_u on the diagonal (als_model.cu:156-159).
@@ -156,26 +157,16 @@ template <int T, int E, bool AUG = true> struct Geo {
 };
 
 // ------------------------------------------------------------------ Gram
-// Zero the stage columns no chunk writes (padding factors past the loaded
-// segments), once per row.
+// Zero the 16-bit stage's columns that no chunk writes (padding factors past
+// the loaded segments), once per row.
 template <int T, int E, bool AUG>
 __device__ __forceinline__ void stage_clear(int f, char *stage) {
     using G = Geo<T, E, AUG>;
-    const int l = lane();
-    if constexpr (E == PREC_FP32) {
-        float *Ys = reinterpret_cast<float *>(stage);
-        const int nseg = (f + 3) >> 2;  // float4 segments carrying data
-        for (int e = l; e < CHUNK * (G::FP - 4 * nseg); e += WAVE) {
-            int k = e / (G::FP - 4 * nseg), col = 4 * nseg + e % (G::FP - 4 * nseg);
-            Ys[k * G::YR + col] = 0.f;
-        }
-    } else {
-        uint16_t *Yt = reinterpret_cast<uint16_t *>(stage);
-        const int nseg = (f + 7) >> 3;  // 16-byte segments carrying data
-        for (int e = l; e < (G::FP - 8 * nseg) * CHUNK; e += WAVE) {
-            int j = 8 * nseg + e / CHUNK, k = e % CHUNK;
-            Yt[G::yt_row(j) * G::YT_H + k] = 0;
-        }
+    uint16_t *Yt = reinterpret_cast<uint16_t *>(stage);
+    const int nseg = (f + 7) >> 3;  // 16-byte segments carrying data
+    for (int e = lane(); e < (G::FP - 8 * nseg) * CHUNK; e += WAVE) {
+        int j = 8 * nseg + e / CHUNK, k = e % CHUNK;
+        Yt[G::yt_row(j) * G::YT_H + k] = 0;
     }
 }
 
@@ -597,6 +588,214 @@ __device__ __forceinline__ void gram_row16_dma(const UpdateArgs &a, int64_t rs, 
                         reinterpret_cast<float *>(stage + 2 * BUF) + 32);
 }
 
+// An FP32 value as the sum of three BF16 ones, each rounded to nearest: h the
+// value, m and l the remainders. x - h - m - l is below 2^-24 |x|. Eight
+// values, as MFMA operands. A remainder x - h is one instruction for either
+// half of a packed pair, a BF16 dot product with (-1, 0) or (0, -1) added to
+// x, exact: neg_lo and neg_hi hold these constants in registers (as a literal
+// -1.0 the second one is not read as a BF16 pair). SAT: h stays finite for
+// values beyond the largest BF16 one (ratings; a factor that large overflows
+// its own square anyway).
+struct Bf16x3 {
+    u32x4 h, m, l;
+};
+template <bool SAT>
+__device__ __forceinline__ Bf16x3 split3(const float (&x)[8], uint32_t neg_lo, uint32_t neg_hi) {
+    typedef float f32x2v __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    const b2 nl = __builtin_bit_cast(b2, neg_lo), nh = __builtin_bit_cast(b2, neg_hi);
+    constexpr float BIG = 3.3895313892515355e38f;  // the largest BF16 value
+    Bf16x3 o;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float x0 = x[2 * w], x1 = x[2 * w + 1];
+        const f32x2v hx = SAT ? f32x2v{__builtin_amdgcn_fmed3f(x0, -BIG, BIG), __builtin_amdgcn_fmed3f(x1, -BIG, BIG)}
+                              : f32x2v{x0, x1};
+        const b2 h = __builtin_convertvector(hx, b2);
+        const float r0 = __builtin_amdgcn_fdot2_f32_bf16(h, nl, x0, false);
+        const float r1 = __builtin_amdgcn_fdot2_f32_bf16(h, nh, x1, false);
+        const b2 m = __builtin_convertvector(f32x2v{r0, r1}, b2);
+        const float s0 = __builtin_amdgcn_fdot2_f32_bf16(m, nl, r0, false);
+        const float s1 = __builtin_amdgcn_fdot2_f32_bf16(m, nh, r1, false);
+        o.h[w] = __builtin_bit_cast(uint32_t, h);
+        o.m[w] = __builtin_bit_cast(uint32_t, m);
+        o.l[w] = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2v{s0, s1}, b2));
+    }
+    return o;
+}
+__device__ __forceinline__ f32x4 mfma_bf16(const u32x4 &a, const u32x4 &b, const f32x4 &c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0,
+                                                   0);
+}
+
+// FP32 Gram of one row on the BF16 matrix pipes. Every FP32 operand is split
+// into three BF16 parts (split3), and a tile takes the six products of them
+// that reach FP32's last bits (hh, hm, mh, mm, hl, lh; what is left out is
+// below 2^-24 of a product): six 16x16x32 MFMAs of 16 cycles for 32 ratings
+// where the FP32 pipe takes eight 16x16x4 ones of 32 cycles. The matrix pipe
+// drops bits as it adds (its sums lean towards zero), so a chunk's products,
+// small ones first, start from zero and the chunk is added to the row's tiles
+// by the VALU, which rounds to nearest: on 3,000 normal ratings the Gram is
+// 0.55 x 2^-24 off in the mean, 1.1 at the worst 3.1 of the FP32 pipe, and 5.3
+// when the chunks accumulate in the matrix pipe.
+// The chunk's rows are gathered by LDS-DMA (as in gram_dma_loop) into one
+// FP32 stage, [rating][factor]; once a chunk's operands are in registers, the
+// next chunk's gathers are issued into the same stage and land while the
+// splits and MFMAs run (one stage: two would leave no room for a second wave
+// per SIMD's at 7 tiles). Load e of the wave fills rows RPL e .. RPL e +
+// RPL - 1 (lane (g, p): 16-byte segment p of row RPL e + g).
+// The contraction over the ratings runs in any order, so lane (q, c) takes
+// ratings 4j + q, j = 0..7, as its eight k: its reads of one j are four
+// consecutive stage rows, which lie 16 LDS banks apart for odd T; for even T
+// the stage holds column block I of row k at block I ^ x(k), x(k) = k % 4
+// (T % 4 == 0) or (k / 2) % 2, which puts them 16 banks apart too.
+// Against the FP32 pipe's form (a chunk gathered through registers, then
+// 16x16x4 MFMAs, nothing in flight meanwhile), one sweep: f = 100 on a quarter
+// of the netflix-shaped users (24.8M ratings) 7.02 -> 3.37 ms; at the ml10M
+// shape f = 100 with CG 3.50 -> 1.23 ms, f = 64 1.50 -> 0.99 ms. The solutions'
+// error against 64 bits fell (1.6e-5 -> 7.9e-6 on the first: the 16x16x32 form
+// rounds its sums less often). At f = 100 the splits issue about 310 VALU
+// instructions and the tiles 168 MFMAs (2,688 busy cycles) a chunk.
+template <int T, bool AUG>
+__device__ __forceinline__ void gram_row32(const UpdateArgs &a, int64_t rs, int n, f32x4 (&acc)[T * (T + 1) / 2],
+                                           float (&bc)[T], char *lds) {
+    using G = Geo<T, PREC_FP32, AUG>;
+    typedef __attribute__((address_space(3))) void lds_void;
+    constexpr int FP = G::FP, NS = FP / 4;  // NS 16-byte segments per row
+    constexpr int RPL = NS <= 4 ? 16 : NS <= 8 ? 8 : NS <= 16 ? 4 : NS <= 32 ? 2 : 1, LPC = CHUNK / RPL;
+    constexpr int XM = T % 4 == 0 ? 4 : T % 2 == 0 ? 2 : 1;  // blocks that x(k) exchanges
+    auto x_of = [](int k) { return T % 4 == 0 ? k & 3 : T % 2 == 0 ? (k >> 1) & 1 : 0; };
+    const int l = lane(), q = l >> 4, c = l & 15;
+    const int f = a.f;
+    int *ib = reinterpret_cast<int *>(lds);
+    float *rb = reinterpret_cast<float *>(lds) + 32;
+    float *st = reinterpret_cast<float *>(lds + G::MISC_FLOATS * 4);
+    if (n <= 0) return;
+    const bool active = l < RPL * NS;
+    const int g = l / NS, p = l - g * NS;
+    int soff[2];  // byte offset of this lane's segment in its row, loads of even and odd e
+    soff[0] = 16 * (p ^ (4 * x_of(g)));
+    soff[1] = 16 * (p ^ (4 * x_of(RPL + g)));
+    int roff[XM];  // block I of row q: roff[I % XM] + 16 (I - I % XM)
+#pragma unroll
+    for (int b = 0; b < XM; ++b) roff[b] = q * FP + 16 * (b ^ x_of(q)) + c;
+    const __amdgpu_buffer_rsrc_t ysr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.Y), (short)0, a.y_bytes, 0x00020000);
+    // index and rating of slot l % 32 of the chunk at k0 (past the row's end: its last rating)
+    auto load_ids = [&](int k0, int &id_raw, float &v_raw) {
+        const int64_t at = rs + min(k0 + (lane_here() & 31), n - 1);
+        id_raw = a.idx[at];
+        v_raw = a.val[at];
+    };
+    // ib[LPC g + e] = index of rating RPL e + g (-1 past the row's end), rb[m] = rating m
+    auto publish = [&](int k0, int id_raw, float v_raw) {
+        const int m = lane_here() & 31;
+        const bool in = k0 + m < n;
+        ib[LPC * (m % RPL) + m / RPL] = in ? id_raw : -1;
+        rb[m] = in ? v_raw : 0.f;
+    };
+    auto dma = [&]() {
+        if (!active) return;
+        const int gi = lane_here() / NS;  // = g, recomputed rather than kept
+#pragma unroll
+        for (int e0 = 0; e0 < LPC; e0 += 4) {
+            int ids[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e0 + e < LPC) ids[e] = ib[LPC * gi + e0 + e];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (e0 + e >= LPC) break;
+                lds_void *dst = (lds_void *)(st + RPL * (e0 + e) * FP);
+                if (a.y_bytes > 0) {
+                    // index -1 wraps to an offset past the buffer: the load touches no memory
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(ysr, dst, 16, ids[e] * (4 * G::LD) + soff[e & 1], 0, 0, 0);
+                } else {
+                    const float *row = ids[e] >= 0 ? a.Y + (int64_t)ids[e] * G::LD : a.zero32;
+                    __builtin_amdgcn_global_load_lds(row + soff[e & 1] / 4, dst, 16, 0, 0);
+                }
+            }
+        }
+    };
+    uint32_t neg_lo = 0x0000bf80u, neg_hi = 0xbf800000u;
+    asm volatile("" : "+v"(neg_lo), "+v"(neg_hi));
+    int id;
+    float v;
+    load_ids(0, id, v);
+    publish(0, id, v);
+    wave_sync();
+    dma();
+    load_ids(CHUNK, id, v);
+    for (int k0 = 0; k0 < n; k0 += CHUNK) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the chunk has landed
+        const int nv = min(CHUNK, n - k0);
+        if (nv < CHUNK) {
+            // rows past the row's end: zero (16-byte pieces; piece e is row nv + e / NS)
+            for (int e = l; e < (CHUNK - nv) * NS; e += WAVE)
+                *reinterpret_cast<f32x4 *>(st + nv * FP + 4 * e) = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if constexpr (AUG) {
+            // the rating into column f (block T - 1, kept at T - 1 ^ x)
+            if (const int k = lane_here(); k < CHUNK)
+                st[k * FP + 16 * ((T - 1) ^ x_of(k)) + (f & 15)] = rb[k];
+        }
+        wave_sync();
+        float F[T][8], r[8];
+#pragma unroll
+        for (int I = 0; I < T; ++I)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) F[I][j] = st[4 * j * FP + roff[I % XM] + 16 * (I - I % XM)];
+        if constexpr (!AUG) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) r[j] = rb[4 * j + q];
+        }
+        // the next chunk into the stage once its operands are in registers
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (k0 + CHUNK < n) {
+            publish(k0 + CHUNK, id, v);
+            wave_sync();
+            dma();
+            load_ids(k0 + 2 * CHUNK, id, v);
+        }
+        if constexpr (AUG) {
+            // whatever a caller's rows hold past column f stays out
+#pragma unroll
+            for (int j = 0; j < 8; ++j) F[T - 1][j] = c <= (f & 15) ? F[T - 1][j] : 0.f;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+#pragma unroll
+                for (int I = 0; I < T; ++I) bc[I] = fmaf(F[I][j], r[j], bc[I]);
+        }
+        Bf16x3 S[T];
+#pragma unroll
+        for (int I = 0; I + 1 < T; ++I) S[I] = split3<false>(F[I], neg_lo, neg_hi);
+        S[T - 1] = split3<AUG>(F[T - 1], neg_lo, neg_hi);
+        // tile (I, J): A = block J, B = block I; four tiles at a time
+#pragma unroll
+        for (int I = 0; I < T; ++I)
+#pragma unroll
+            for (int J0 = 0; J0 <= I; J0 += 4) {
+                f32x4 z[4];
+                auto each = [&](auto fn) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (J0 + t <= I) z[t] = fn(S[J0 + t], z[t]);
+                };
+                each([&](const Bf16x3 &j, const f32x4 &) { return mfma_bf16(j.l, S[I].h, f32x4{0.f, 0.f, 0.f, 0.f}); });
+                each([&](const Bf16x3 &j, const f32x4 &y) { return mfma_bf16(j.h, S[I].l, y); });
+                each([&](const Bf16x3 &j, const f32x4 &y) { return mfma_bf16(j.m, S[I].m, y); });
+                each([&](const Bf16x3 &j, const f32x4 &y) { return mfma_bf16(j.m, S[I].h, y); });
+                each([&](const Bf16x3 &j, const f32x4 &y) { return mfma_bf16(j.h, S[I].m, y); });
+                each([&](const Bf16x3 &j, const f32x4 &y) { return mfma_bf16(j.h, S[I].h, y); });
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (J0 + t <= I) acc[tile_id(I, J0 + t)] += z[t];
+            }
+        wave_sync();
+    }
+}
+
 // The Gram of ratings rs .. rs + n - 1 of a row; with AUG = false also b, in
 // column form, each lane row q holding its share of the ratings (q4_sum adds
 // them). With AUG, b is row f of the tiles.
@@ -621,30 +820,14 @@ __device__ __forceinline__ void gram_row(const UpdateArgs &a, int64_t rs, int n,
         gram_row16_piped<T, E, AUG>(a, rs, n, acc, bc, lds);
         return;
     }
-    if constexpr (AUG) stage_clear<T, E, AUG>(a.f, stage);
-    for (int k0 = 0; k0 < n; k0 += CHUNK) {
-        stage_chunk<T, E, AUG>(a, rs, k0, min(CHUNK, n - k0), lds);
-        if constexpr (E == PREC_FP32) {
-            const float *Ys = reinterpret_cast<const float *>(stage);
-            const float *rbuf = reinterpret_cast<const float *>(lds) + 32;
-#pragma unroll
-            for (int ks = 0; ks < CHUNK / 4; ++ks) {
-                float F[T];
-#pragma unroll
-                for (int I = 0; I < T; ++I) F[I] = Ys[(4 * ks + (l >> 4)) * G::YR + 16 * I + (l & 15)];
-                if constexpr (!AUG) {
-                    const float r = rbuf[4 * ks + (l >> 4)];
-#pragma unroll
-                    for (int I = 0; I < T; ++I) bc[I] = fmaf(F[I], r, bc[I]);
-                }
-#pragma unroll
-                for (int I = 0; I < T; ++I)
-#pragma unroll
-                    for (int J = 0; J <= I; ++J)
-                        acc[tile_id(I, J)] =
-                            __builtin_amdgcn_mfma_f32_16x16x4f32(F[J], F[I], acc[tile_id(I, J)], 0, 0, 0);
-            }
-        } else {
+    if constexpr (E == PREC_FP32) {
+        gram_row32<T, AUG>(a, rs, n, acc, bc, lds);
+        return;
+    }
+    if constexpr (E != PREC_FP32 && T > 8) {
+        stage_clear<T, E, AUG>(a.f, stage);
+        for (int k0 = 0; k0 < n; k0 += CHUNK) {
+            stage_chunk<T, E, AUG>(a, rs, k0, min(CHUNK, n - k0), lds);
             const uint16_t *Yt = reinterpret_cast<const uint16_t *>(stage);
             u32x4 F[T];
 #pragma unroll
@@ -655,16 +838,14 @@ __device__ __forceinline__ void gram_row(const UpdateArgs &a, int64_t rs, int n,
 #pragma unroll
                 for (int J = 0; J <= I; ++J) {
                     if constexpr (E == PREC_BF16)
-                        acc[tile_id(I, J)] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                            __builtin_bit_cast(bf16x8, F[J]), __builtin_bit_cast(bf16x8, F[I]), acc[tile_id(I, J)],
-                            0, 0, 0);
+                        acc[tile_id(I, J)] = mfma_bf16(F[J], F[I], acc[tile_id(I, J)]);
                     else
                         acc[tile_id(I, J)] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                             __builtin_bit_cast(f16x8, F[J]), __builtin_bit_cast(f16x8, F[I]), acc[tile_id(I, J)],
                             0, 0, 0);
                 }
+            wave_sync();
         }
-        wave_sync();
     }
 }
 
@@ -1838,8 +2019,13 @@ __device__ __forceinline__ void update_body(const UpdateArgs &a) {
     }
 }
 
+// FP32 systems of up to 7 blocks are held to two waves per SIMD: with CG at 7
+// blocks the compiler would otherwise take 282 registers, and one wave alone
+// has nothing to run under its gathers.
 template <int T, int E, int S, bool AUG>
-__global__ __launch_bounds__(WAVE) void update_kernel(UpdateArgs a) {
+__global__ __launch_bounds__(WAVE)
+__attribute__((amdgpu_waves_per_eu(E == PREC_FP32 && S != SOLVE_CHOL_WARM && T <= 7 ? 2 : 1))) void update_kernel(
+    UpdateArgs a) {
     update_body<T, E, S, AUG>(a);
 }
 

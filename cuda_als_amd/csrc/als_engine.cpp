@@ -281,6 +281,7 @@ UpdateArgs side_args(als_engine *e, const Side &s, const float *Y, const uint16_
         const int64_t ny = &s == &e->side[0] ? e->n : e->m;  // rows of Y
         const int64_t bytes = ny * e->ld * (int64_t)sizeof(uint16_t);
         a.ys_bytes = bytes <= INT32_MAX ? (int)bytes : 0;
+        a.y_bytes = 2 * bytes <= INT32_MAX ? (int)(2 * bytes) : 0;
     }
     a.gram_dma = s.gram_dma;
     return a;

@@ -63,6 +63,7 @@ struct UpdateArgs {
     const uint16_t *zero16;     // same, 16-bit
     int ys_bytes;               // bytes of the 16-bit Y shadow when below 2^31 (the pipelined
                                 // Gram then gathers with 32-bit buffer offsets), else 0
+    int y_bytes;                // bytes of Y when below 2^31 (the FP32 Gram's gathers), else 0
     int gram_dma;               // 1: the 16-bit Gram gathers straight to LDS where built
                                 // (gram_dma_built), 0: through registers
 };

@@ -41,7 +41,7 @@ SOLVES = {"chol": (E.SolveType.CHOL, 0, False), "warm": (E.SolveType.CHOL, 1, Tr
 # parts of split rows refine against the 16-bit system, so the refined solver runs unsplit
 @pytest.mark.parametrize("solve,split_len", [(s, n) for s in SOLVES for n in (0, 40) if (s, n) != ("refined", 40)])
 @pytest.mark.parametrize("prec", list(ORACLE_PREC))
-@pytest.mark.parametrize("f", [15, 16, 17, 32, 48, 63, 64, 65, 80, 96, 112, 127, 128, 129])
+@pytest.mark.parametrize("f", [15, 16, 17, 32, 40, 48, 63, 64, 65, 80, 90, 96, 100, 112, 127, 128, 129, 143])
 def test_half_sweep(f, prec, solve, split_len):
     """Within 1e-4 of the FP64 oracle, as the other half-sweep tests ask (the
     oracle's system is formed from the same rounded factors, so the precision
@@ -92,3 +92,31 @@ def test_padding_of_caller_buffers(f, prec):
         torch.cuda.synchronize()
         for t in (X, xbar, ybar):
             assert not t[:, f:].any() and t[:, :f].any()
+
+
+def test_fp32_factors_beyond_two_gib():
+    """A fixed side past 2 GiB takes the FP32 Gram's 64-bit addresses instead
+    of buffer offsets: users whose items lie at both ends of it, against the
+    oracle (bar as above)."""
+    import torch
+    f, n = 100, (1 << 31) // (4 * 112) + 1000
+    rng = np.random.default_rng(3)
+    near = np.concatenate([np.arange(150), np.arange(n - 150, n)])
+    lengths = [1, 31, 90, 200, 300]
+    pos = np.concatenate([np.sort(rng.choice(near.size, k, replace=False)) for k in lengths])
+    val = rng.integers(1, 6, pos.size).astype(np.float32)
+    ptr = np.concatenate([[0], np.cumsum(lengths)])
+    d = ca.from_arrays(len(lengths), n, ptr, near[pos], val, [0], [0], [3.0])
+    V0 = (0.4 * rng.standard_normal((near.size, f))).astype(np.float32)
+    want = O.update_rows(O.config(f, 0.05, O.SOLVE_CHOL), np.arange(len(lengths)), ptr, pos, val, V0.astype(np.float64))
+    with E.Engine(E.make_config(f, 0.05, 1, E.SolveType.CHOL, E.Prec.FP32), d) as e:
+        class Rows:
+            __cuda_array_interface__ = {"shape": (n, 112), "typestr": "<f4", "version": 3, "strides": None,
+                                        "data": (e.device_factors(ca.ALS_SIDE_ITEMS), False)}
+        Y = torch.as_tensor(Rows(), device="cuda")
+        Y[torch.as_tensor(near, device="cuda"), :f] = torch.as_tensor(V0, device="cuda")
+        torch.cuda.synchronize()
+        e.set_dual_limit(ca.ALS_SIDE_USERS, 0)
+        e.update(ca.ALS_SIDE_USERS)
+        got = e.get_factors(ca.ALS_SIDE_USERS)
+    assert rel(got, want) <= 1e-4
