@@ -10,7 +10,8 @@
 //   * units are ordered by decreasing cost (longest-processing-time first),
 //     so the tail of the launch is made of the lightest rows;
 //   * consecutive units are grouped into batches of about `batch_work`
-//     rating-equivalents; persistent waves pop batches from a device queue.
+//     rating-equivalents, where those would be small larger ones first;
+//     persistent waves take batches from a device queue.
 #pragma once
 #include <cstdint>
 #include <vector>
