@@ -1519,6 +1519,35 @@ __device__ __forceinline__ float colform_dot(const float *a, const float *b, int
 }
 
 // ------------------------------------------------------------ mat-vec
+// Sums of four values over the 16 lanes of a row, scattered: lane c gets
+// the total of v[c & 3] (the FP32 form of rows16_scatter_d).
+__device__ __forceinline__ float rows16_scatter4(const f32x4 &v) {
+    const int c = lane() & 15;
+    const bool b1 = (c & 2) != 0, b0 = (c & 1) != 0;
+    const float u0 = (b1 ? v[2] : v[0]) + dpp_mov<0x4E>(b1 ? v[0] : v[2]);
+    const float u1 = (b1 ? v[3] : v[1]) + dpp_mov<0x4E>(b1 ? v[1] : v[3]);
+    float t = (b0 ? u1 : u0) + dpp_mov<0xB1>(b0 ? u0 : u1);
+    t += dpp_mov<0x124>(t);
+    t += dpp_mov<0x128>(t);
+    return t;
+}
+
+// Column-form vector -> one row of a factor matrix in global memory
+// (row-group q stores blocks q, q+4, ...; 16 consecutive floats each). PAD:
+// a block of zeros follows (the matrices' stride is the augmented system's).
+template <int T, bool PAD = false>
+__device__ __forceinline__ void store_colform(float *dst, const float (&v)[T]) {
+    const int l = lane(), q = l >> 4, c = l & 15;
+#pragma unroll
+    for (int J4 = 0; J4 < T + PAD; J4 += 4) {
+        const int J = J4 + q;
+        float val = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (J4 + k < T && q == k) val = v[J4 + k];
+        if (J < T + PAD) dst[16 * J + c] = val;
+    }
+}
 // y = A v for the symmetric matrix held as tiles (layout above, before any
 // factorisation), restricted to the leading f x f block. v and y in column
 // form (zero past f).
@@ -1530,38 +1559,48 @@ __device__ __forceinline__ float colform_dot(const float *a, const float *b, int
 // are complete at the end of step J, so y[J] is formed there and only one
 // row-form partial and one row form of v are live at a time. Each partial
 // sums its terms in ascending block order.
+// v's row forms are read from vs (16T floats of this wave's LDS), one 16-byte
+// read a block behind one round of writes, and a block's row-form sums are
+// scattered over the lanes and moved by one shuffle: with four shuffles for
+// the row form and four full sums over 16 lanes a block, as before, the
+// exchanges were half of the mat-vec's instructions. One sweep at the ml10M
+// shape: f = 100 FP32 1.274 -> 1.261 ms, f = 80 with the 16-bit Gram 0.585 ->
+// 0.580 ms; 8,192 batched systems of f = 100 100.9 -> 99.8 us (waiting for
+// their matrices, and the rows for their gathers, is most of the rest).
 template <int T, int NT>
-__device__ __forceinline__ void matvec_f32(const f32x4 (&A)[NT], int f, const float (&v)[T], float (&y)[T]) {
-    const int c = lane() & 15;
+__device__ __forceinline__ void matvec_f32(const f32x4 (&A)[NT], int f, const float (&v)[T], float (&y)[T],
+                                           float *vs) {
+    const int l = lane(), q = l >> 4, c = l & 15;
+    store_colform<T>(vs, v);
+    wave_sync();
     float pc[T];
 #pragma unroll
     for (int I = 0; I < T; ++I) pc[I] = 0.f;
 #pragma unroll
     for (int J = 0; J < T; ++J) {
-        const f32x4 vr = col_to_row(v[J]);
-        f32x4 pr = f32x4{0.f, 0.f, 0.f, 0.f};
-        pr += A[tile_id(J, J)] * v[J];
+        const f32x4 vr = *reinterpret_cast<const f32x4 *>(vs + 16 * J + 4 * q);
+        f32x4 pr = A[tile_id(J, J)] * v[J];
 #pragma unroll
         for (int I = J + 1; I < T; ++I) {
             const f32x4 t = A[tile_id(I, J)];
             pc[I] += t[0] * vr[0] + t[1] * vr[1] + t[2] * vr[2] + t[3] * vr[3];
             pr += t * v[I];
         }
-        f32x4 s;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[r] = row16_sum(pr[r]);
-        const float yc = row_to_col(s) + q4_sum(pc[J]);
+        // row 16J + c: lane (c / 4, c) holds the total for register c % 4 of row c / 4
+        const float s = rows16_scatter4(pr);
+        const float yc = __shfl(s, ((c >> 2) << 4) | c, WAVE) + q4_sum(pc[J]);
         y[J] = (16 * J + c < f) ? yc : 0.f;
     }
+    wave_sync();  // vs read before the next product's writes
 }
 
 // cuMF CG (cumf_als_cg/cg.cu:37-232) on the register tiles: warm start x,
 // `iters` iterations, exit when r.r < tol after an update; p.Ap == 0 stops.
 template <int T, int NT>
 __device__ __forceinline__ void cg_regs(const f32x4 (&A)[NT], int f, const float (&b)[T], float (&x)[T], int iters,
-                                        float tol) {
+                                        float tol, float *vs) {
     float r[T], p[T], ap[T];
-    matvec_f32<T>(A, f, x, ap);
+    matvec_f32<T>(A, f, x, ap, vs);
 #pragma unroll
     for (int J = 0; J < T; ++J) {
         r[J] = b[J] - ap[J];
@@ -1569,7 +1608,7 @@ __device__ __forceinline__ void cg_regs(const f32x4 (&A)[NT], int f, const float
     }
     float rsold = colform_dot(r, r, T);
     for (int it = 0; it < iters; ++it) {
-        matvec_f32<T>(A, f, p, ap);
+        matvec_f32<T>(A, f, p, ap, vs);
         const float pap = colform_dot(p, ap, T);
         if (pap == 0.f) break;
         const float alpha = rsold / pap;
@@ -1589,22 +1628,6 @@ __device__ __forceinline__ void cg_regs(const f32x4 (&A)[NT], int f, const float
     }
 }
 
-// Column-form vector -> one row of a factor matrix in global memory
-// (row-group q stores blocks q, q+4, ...; 16 consecutive floats each). PAD:
-// a block of zeros follows (the matrices' stride is the augmented system's).
-template <int T, bool PAD = false>
-__device__ __forceinline__ void store_colform(float *dst, const float (&v)[T]) {
-    const int l = lane(), q = l >> 4, c = l & 15;
-#pragma unroll
-    for (int J4 = 0; J4 < T + PAD; J4 += 4) {
-        const int J = J4 + q;
-        float val = 0.f;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-            if (J4 + k < T && q == k) val = v[J4 + k];
-        if (J < T + PAD) dst[16 * J + c] = val;
-    }
-}
 template <int T, int E>
 __device__ __forceinline__ void store_colform16(uint16_t *dst, const float (&v)[T]) {
     const int l = lane(), q = l >> 4, c = l & 15;
@@ -1668,19 +1691,6 @@ __device__ __forceinline__ float rows16_scatter8(const float (&v)[8]) {
     for (int i = 0; i < 2; ++i) t[i] = (b2 ? u[2 + i] : u[i]) + dpp_mov<0x141>(b2 ? u[i] : u[2 + i]);
     float z = (b1 ? t[1] : t[0]) + dpp_mov<0x4E>(b1 ? t[0] : t[1]);
     return z + dpp_mov<0xB1>(z);
-}
-
-// Sums of four values over the 16 lanes of a row, scattered: lane c gets
-// the total of v[c & 3] (the FP32 form of rows16_scatter_d).
-__device__ __forceinline__ float rows16_scatter4(const float (&v)[4]) {
-    const int c = lane() & 15;
-    const bool b1 = (c & 2) != 0, b0 = (c & 1) != 0;
-    const float u0 = (b1 ? v[2] : v[0]) + dpp_mov<0x4E>(b1 ? v[0] : v[2]);
-    const float u1 = (b1 ? v[3] : v[1]) + dpp_mov<0x4E>(b1 ? v[1] : v[3]);
-    float t = (b0 ? u1 : u0) + dpp_mov<0xB1>(b0 ? u0 : u1);
-    t += dpp_mov<0x124>(t);
-    t += dpp_mov<0x128>(t);
-    return t;
 }
 
 // Operands of the dual Gram, one step of the factor dimension: lane (q, c)
@@ -1793,7 +1803,7 @@ __device__ __forceinline__ void dual_row(const UpdateArgs &a, int64_t rs, int n,
         dual_operands<TD, T, E, AUG>(a, id, s, nseg, F);
         const int seg = 4 * s + q;
         if constexpr (E == PREC_FP32) {
-            float p[4] = {0.f, 0.f, 0.f, 0.f};
+            f32x4 p = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int I = 0; I < TD; ++I)
 #pragma unroll
@@ -1991,7 +2001,7 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                             for (int r = 0; r < 4; ++r) acc[t][r] = (float)(_Float16)acc[t][r];
                     }
                     load_colform<T>(a.X + (int64_t)row * G::LD, f, x);
-                    cg_regs<T>(acc, f, bv, x, a.cg_iters, a.cg_tol);
+                    cg_regs<T>(acc, f, bv, x, a.cg_iters, a.cg_tol, xs);
                 }
                 bool finite = true;
 #pragma unroll
