@@ -329,7 +329,7 @@ __global__ __launch_bounds__(WAVE) void adjoint_solve_kernel(AdjointArgs a) {
             f32x4 L[NT];
             const float *src = a.Lsave + (int64_t)row * NT * 256;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) L[t] = *reinterpret_cast<const f32x4 *>(src + t * 256 + 4 * l);
+            for (int t = 0; t < NT; ++t) L[t] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(src + t * 256 + 4 * l));
             load_colform<T>(a.Gbar + o, f, g);
             f32x4 wr[T];
             fwd_solve<T>(L, f, g, wr);
