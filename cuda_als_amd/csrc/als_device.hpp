@@ -113,6 +113,7 @@ template <int T, int E, bool AUG = true> struct Geo {
     static constexpr int FP = 16 * T;           // padded dimension of the system
     // Row stride of the factor matrices: always that of the augmented system
     static constexpr int LD = AUG ? FP : FP + 16;
+    static constexpr int SH = shadow_stride_tiles(T);  // row stride of the 16-bit shadows (halves)
     // Floats of one part of a split row: the tiles and, where it is not in
     // them, b
     static constexpr int PART = NT * 256 + (AUG ? 0 : FP);
@@ -221,7 +222,7 @@ __device__ __forceinline__ void stage_chunk(const UpdateArgs &a, int64_t rs, int
                 // Unused slots of the last chunk read a row of zeros: the
                 // load itself is unconditional.
                 const int id = ibuf[8 * g + e];
-                const uint16_t *src = id >= 0 ? Ysh + (int64_t)id * G::LD + 8 * s : a.zero16 + 8 * s;
+                const uint16_t *src = id >= 0 ? Ysh + (int64_t)id * G::SH + 8 * s : a.zero16 + 8 * s;
                 d[e] = *reinterpret_cast<const u32x4 *>(src);
             }
 #pragma unroll
@@ -345,16 +346,16 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
             const int ids[8] = {i0.x, i0.y, i0.z, i0.w, i1.x, i1.y, i1.z, i1.w};
             if (a.ys_bytes > 0) {
                 // Buffer loads with a 32-bit byte offset: a slot past the
-                // row's end (id -1) has an offset of 2^32 - 2 LD + 2 soff,
+                // row's end (id -1) has an offset of 2^32 - 2 SH + 2 soff,
                 // beyond the buffer, and reads zeros.
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     d[e] = __builtin_bit_cast(
-                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(ysr, ids[e] * (2 * G::LD) + soff2, 0, 0));
+                        u32x4, __builtin_amdgcn_raw_buffer_load_b128(ysr, ids[e] * (2 * G::SH) + soff2, 0, 0));
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    const uint16_t *src = (ids[e] >= 0 ? a.Ys + (int64_t)ids[e] * G::LD : a.zero16) + soff;
+                    const uint16_t *src = (ids[e] >= 0 ? a.Ys + (int64_t)ids[e] * G::SH : a.zero16) + soff;
                     d[e] = *reinterpret_cast<const u32x4 *>(src);
                 }
             }
@@ -497,7 +498,7 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
 #pragma unroll
             for (int e = 0; e < 8; ++e)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(ysr, (lds_void *)(dst + 4 * e * RS), 16,
-                                                         ids[e] * (2 * G::LD) + soff2, 0, 0, 0);
+                                                         ids[e] * (2 * G::SH) + soff2, 0, 0, 0);
         }
     };
     using P0 = std::integral_constant<int, 0>;
@@ -1712,7 +1713,7 @@ __device__ __forceinline__ void dual_operands(const UpdateArgs &a, const int (&i
             if constexpr (E == PREC_FP32)
                 F[I] = *reinterpret_cast<const u32x4 *>(a.Y + (int64_t)id[I] * G::LD + SEGW * seg);
             else
-                F[I] = *reinterpret_cast<const u32x4 *>(a.Ys + (int64_t)id[I] * G::LD + SEGW * seg);
+                F[I] = *reinterpret_cast<const u32x4 *>(a.Ys + (int64_t)id[I] * G::SH + SEGW * seg);
         }
     }
 }
@@ -2019,7 +2020,7 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
             }
             store_colform<T, !AUG>(a.X + (int64_t)row * G::LD, x);
             if constexpr (E != PREC_FP32) {
-                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::LD, x);
+                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::SH, x);
             }
         }
     }
@@ -2078,7 +2079,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(4, 4))) vo
             }
             store_colform<T, !AUG>(a.X + (int64_t)row * G::LD, x);
             if constexpr (E != PREC_FP32) {
-                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::LD, x);
+                if (a.Xs) store_colform16<T, E>(a.Xs + (int64_t)row * G::SH, x);
             }
         }
     }

@@ -54,7 +54,7 @@ struct Side {
 
 struct als_engine {
     als_config cfg{};
-    int T = 0, ld = 0, prec = PREC_FP32, solve = SOLVE_CHOL, lds = 0;
+    int T = 0, ld = 0, sh = 0, prec = PREC_FP32, solve = SOLVE_CHOL, lds = 0;
     int dual_max = 0, dual_lds = 0, dual_grid = 0;  // dual kernel: rows below dual_max ratings (0: none)
     int grid_v1 = 0;                                  // persistent waves of the variant-1 kernel (0: none)
     int grid_max = 0;                                 // occupancy limit of the default update kernel
@@ -279,9 +279,9 @@ UpdateArgs side_args(als_engine *e, const Side &s, const float *Y, const uint16_
     a.zero16 = e->zero16;
     {
         const int64_t ny = &s == &e->side[0] ? e->n : e->m;  // rows of Y
-        const int64_t bytes = ny * e->ld * (int64_t)sizeof(uint16_t);
-        a.ys_bytes = bytes <= INT32_MAX ? (int)bytes : 0;
-        a.y_bytes = 2 * bytes <= INT32_MAX ? (int)(2 * bytes) : 0;
+        const int64_t sb = ny * e->sh * (int64_t)sizeof(uint16_t), yb = ny * e->ld * (int64_t)sizeof(float);
+        a.ys_bytes = sb <= INT32_MAX ? (int)sb : 0;
+        a.y_bytes = yb <= INT32_MAX ? (int)yb : 0;
     }
     a.gram_dma = s.gram_dma;
     return a;
@@ -398,7 +398,7 @@ int refresh_shadow(als_engine *e, int sd) {
     const int64_t rows = sd == 0 ? e->m : e->n;
     const float *src = sd == 0 ? e->U : e->V;
     uint16_t *dst = sd == 0 ? e->Us : e->Vs;
-    HIPCHK(e, launch_to16(e->prec, src, dst, rows * e->ld, e->stream));
+    HIPCHK(e, launch_to16(e->cfg.f, e->prec, src, dst, rows, e->stream));
     return ALS_OK;
 }
 
@@ -453,7 +453,8 @@ int als_create(const als_config *cfg, als_engine **out) {
     auto *e = new als_engine;
     e->cfg = *cfg;
     e->T = blocks_for_T(cfg->f);
-    e->ld = 16 * e->T;
+    e->ld = row_stride(cfg->f);
+    e->sh = shadow_stride(cfg->f);
     e->prec = cfg->gram_prec;
     e->solve = (cfg->solve_type == ALS_SOLVE_CG_FP32 || cfg->solve_type == ALS_SOLVE_CG_FP16) ? SOLVE_CG
                : cfg->refine_steps == 1 && cfg->refine_warm                               ? SOLVE_CHOL_WARM
@@ -585,7 +586,7 @@ int als_set_train(als_engine *e, int64_t m, int64_t n, int64_t nnz, const int *c
         (rc = dev_alloc(e, &e->coo_row, nnz)) ||
         (rc = dev_alloc(e, &e->U, m * e->ld)) || (rc = dev_alloc(e, &e->V, n * e->ld)))
         return rc;
-    if (e->prec != PREC_FP32 && ((rc = dev_alloc(e, &e->Us, m * e->ld)) || (rc = dev_alloc(e, &e->Vs, n * e->ld))))
+    if (e->prec != PREC_FP32 && ((rc = dev_alloc(e, &e->Us, m * e->sh)) || (rc = dev_alloc(e, &e->Vs, n * e->sh))))
         return rc;
     HIPCHK(e, hipMemcpyAsync(su.ptr, csr_ptr, (m + 1) * sizeof(int), hipMemcpyHostToDevice, e->stream));
     HIPCHK(e, hipMemcpyAsync(si.ptr, csc_ptr, (n + 1) * sizeof(int), hipMemcpyHostToDevice, e->stream));
@@ -602,8 +603,8 @@ int als_set_train(als_engine *e, int64_t m, int64_t n, int64_t nnz, const int *c
     }
     HIPCHK(e, hipMemsetAsync(e->U, 0, (size_t)std::max<int64_t>(1, m * e->ld) * sizeof(float), e->stream));
     HIPCHK(e, hipMemsetAsync(e->V, 0, (size_t)std::max<int64_t>(1, n * e->ld) * sizeof(float), e->stream));
-    if (e->Us) HIPCHK(e, hipMemsetAsync(e->Us, 0, (size_t)std::max<int64_t>(1, m * e->ld) * 2, e->stream));
-    if (e->Vs) HIPCHK(e, hipMemsetAsync(e->Vs, 0, (size_t)std::max<int64_t>(1, n * e->ld) * 2, e->stream));
+    if (e->Us) HIPCHK(e, hipMemsetAsync(e->Us, 0, (size_t)std::max<int64_t>(1, m * e->sh) * 2, e->stream));
+    if (e->Vs) HIPCHK(e, hipMemsetAsync(e->Vs, 0, (size_t)std::max<int64_t>(1, n * e->sh) * 2, e->stream));
     e->hptr[0].assign(csr_ptr, csr_ptr + m + 1);
     e->hptr[1].assign(csc_ptr, csc_ptr + n + 1);
     for (int sd = 0; sd < 2; ++sd) {  // the adjoint's parts follow the rating lists
@@ -883,13 +884,13 @@ int forward_impl(als_engine *e, int sd, const float *d_Y, float *d_X, const floa
     int rc = ALS_OK;
     const uint16_t *Ys = nullptr;
     if (e->prec != PREC_FP32) {
-        size_t need = (size_t)std::max<int64_t>(1, cols * e->ld) * 2;
+        size_t need = (size_t)std::max<int64_t>(1, cols * e->sh) * 2;
         if (e->tmp16_bytes < need) {
             dev_free(e, e->tmp16);
             if ((rc = dev_alloc(e, &e->tmp16, need / 2))) return rc;
             e->tmp16_bytes = need;
         }
-        HIPCHK(e, launch_to16(e->prec, d_Y, e->tmp16, cols * e->ld, e->stream));
+        HIPCHK(e, launch_to16(e->cfg.f, e->prec, d_Y, e->tmp16, cols, e->stream));
         Ys = e->tmp16;
     }
     return launch_side(e, sd, d_Y, Ys, d_X, nullptr, d_lambda_rows, Ls, e->stream);
@@ -1152,19 +1153,19 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
         // save what a trial overwrites
         float *X = sd == 0 ? e->U : e->V;
         uint16_t *Xs = sd == 0 ? e->Us : e->Vs;
-        const size_t cnt = (size_t)std::max<int64_t>(1, rows * e->ld);
+        const size_t cnt = (size_t)std::max<int64_t>(1, rows * e->ld), scnt = (size_t)std::max<int64_t>(1, rows * e->sh);
         float *xsave = nullptr;
         uint16_t *xssave = nullptr;
         int *fsave = nullptr;
-        if ((rc = dev_alloc(e, &xsave, cnt)) || (Xs && (rc = dev_alloc(e, &xssave, cnt))) ||
+        if ((rc = dev_alloc(e, &xsave, cnt)) || (Xs && (rc = dev_alloc(e, &xssave, scnt))) ||
             (rc = dev_alloc(e, &fsave, 1)))
             break;
         HIPCHK(e, hipMemcpyAsync(xsave, X, cnt * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
-        if (Xs) HIPCHK(e, hipMemcpyAsync(xssave, Xs, cnt * 2, hipMemcpyDeviceToDevice, e->stream));
+        if (Xs) HIPCHK(e, hipMemcpyAsync(xssave, Xs, scnt * 2, hipMemcpyDeviceToDevice, e->stream));
         HIPCHK(e, hipMemcpyAsync(fsave, e->fail, sizeof(int), hipMemcpyDeviceToDevice, e->stream));
         auto restore = [&]() -> int {
             HIPCHK(e, hipMemcpyAsync(X, xsave, cnt * sizeof(float), hipMemcpyDeviceToDevice, e->stream));
-            if (Xs) HIPCHK(e, hipMemcpyAsync(Xs, xssave, cnt * 2, hipMemcpyDeviceToDevice, e->stream));
+            if (Xs) HIPCHK(e, hipMemcpyAsync(Xs, xssave, scnt * 2, hipMemcpyDeviceToDevice, e->stream));
             HIPCHK(e, hipMemcpyAsync(e->fail, fsave, sizeof(int), hipMemcpyDeviceToDevice, e->stream));
             return ALS_OK;
         };

@@ -294,17 +294,29 @@ hipError_t launch_rmse(const RmseArgs &a, int blocks, double *out, bool with_rms
 // Gram (float2half_array, als_model.cu:54-60, 1883-1889). Here the update
 // kernel refreshes the shadow as it writes each row; this kernel builds it
 // after factors are set from the host.
-template <int E>
-__global__ void to16_kernel(const float *src, uint16_t *dst, int64_t count) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-        dst[i] = to16<E>(src[i]);
+template <int E, class INT>
+__global__ void to16_kernel(const float *src, uint16_t *dst, INT count, int width, int ld, int sh) {
+    for (INT i = (INT)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (INT)gridDim.x * blockDim.x) {
+        const INT row = i / width;
+        const int j = (int)(i - row * width);
+        dst[(int64_t)row * sh + j] = to16<E>(src[(int64_t)row * ld + j]);
+    }
 }
 
-hipError_t launch_to16(int prec, const float *src, uint16_t *dst, int64_t count, hipStream_t s) {
+template <int E>
+static void to16_rows(int f, const float *src, uint16_t *dst, int64_t rows, hipStream_t s) {
+    const int width = 16 * tiles(f), ld = row_stride(f), sh = shadow_stride(f);
+    const int64_t count = rows * width;
     const int blocks = (int)std::min<int64_t>((count + 255) / 256, 65536);
-    if (count == 0) return hipSuccess;
-    if (prec == PREC_BF16) to16_kernel<PREC_BF16><<<blocks, 256, 0, s>>>(src, dst, count);
-    else if (prec == PREC_FP16) to16_kernel<PREC_FP16><<<blocks, 256, 0, s>>>(src, dst, count);
+    // 32-bit divisions where a thread's last index plus one stride of the grid still fits
+    if (count < (int64_t)1 << 31) to16_kernel<E, uint32_t><<<blocks, 256, 0, s>>>(src, dst, (uint32_t)count, width, ld, sh);
+    else to16_kernel<E, int64_t><<<blocks, 256, 0, s>>>(src, dst, count, width, ld, sh);
+}
+
+hipError_t launch_to16(int f, int prec, const float *src, uint16_t *dst, int64_t rows, hipStream_t s) {
+    if (rows == 0) return hipSuccess;
+    if (prec == PREC_BF16) to16_rows<PREC_BF16>(f, src, dst, rows, s);
+    else if (prec == PREC_FP16) to16_rows<PREC_FP16>(f, src, dst, rows, s);
     else return hipErrorInvalidValue;
     return hipGetLastError();
 }

@@ -22,9 +22,20 @@ constexpr int MAX_T = 9;  // augmented dimension f + 1 <= 16 * MAX_T
 // warm-started BF16 models of f = 32, 64, 128 together 3.25 -> 2.79 ms.
 constexpr int tiles(int f) { return (f + 15) / 16; }
 constexpr bool augmented(int f) { return f % 16 != 0; }
-// Row stride (floats, or halves of the 16-bit shadow) of every factor matrix:
-// the augmented system's, whatever the solve uses.
+// Row stride (floats) of every factor matrix: the augmented system's, whatever
+// the solve uses.
 constexpr int row_stride(int f) { return 16 * ((f + 16) / 16); }
+// Row stride (halves) of the 16-bit shadows, which only the kernels see: 16T,
+// rounded up to a multiple of 64 bytes above one block, so that a row touches
+// as few 128-byte cache lines as its length allows. The rows are gathered in
+// the order of the ratings, and what a gather costs is its lines: reading rows
+// of random users (480,189 of them) took 0.724 ms at 224 bytes a row (f = 100,
+// 2.5 lines) and 0.579 at 256 (2 lines), 0.486 at 160 bytes (f = 64 in an
+// augmented row's stride) and 0.312 at 128, 0.855 at 288 (f = 128) and 0.580
+// at 256. One sweep: the netflix shape, mixed, f = 100 6.79 -> 6.42 ms; three
+// BF16 models of f = 32, 64, 128 at the ml10M shape 2.31 -> 2.26 ms.
+constexpr int shadow_stride_tiles(int T) { return 16 * T + (T > 1 && T % 2 == 1 ? 16 : 0); }
+constexpr int shadow_stride(int f) { return shadow_stride_tiles(tiles(f)); }
 // Floats of one part of a split row or of one copy of a system: its tiles,
 // and b where it is not in them.
 constexpr int part_floats(int f) { return tiles(f) * (tiles(f) + 1) / 2 * 256 + (augmented(f) ? 0 : f); }
@@ -36,9 +47,9 @@ struct UpdateArgs {
     const int *idx;
     const float *val;
     const float *Y;             // fixed factors, FP32, row stride row_stride(f)
-    const uint16_t *Ys;         // fixed factors, 16-bit shadow, the same stride (16-bit Gram only)
+    const uint16_t *Ys;         // fixed factors, 16-bit shadow, row stride shadow_stride(f) (16-bit Gram only)
     float *X;                   // updated factors, FP32, the same stride (CG: warm start in)
-    uint16_t *Xs;               // 16-bit shadow of X to refresh (nullable)
+    uint16_t *Xs;               // 16-bit shadow of X to refresh, the shadows' stride (nullable)
     const float *lambda_rows;   // per-row lambda (nullable -> lambda)
     float lambda;
     int f;
@@ -154,6 +165,7 @@ hipError_t launch_ybar(const YbarArgs &a, hipStream_t s);
 // (blocks doubles), then out[0] = their sum (with_rmse: out[1] = sqrt(sum / n)).
 constexpr int RMSE_BLOCKS = 1024;
 hipError_t launch_rmse(const RmseArgs &a, int blocks, double *out, bool with_rmse, hipStream_t s);
-hipError_t launch_to16(int prec, const float *src, uint16_t *dst, int64_t count, hipStream_t s);
+// The 16-bit shadow of `rows` factor rows (row_stride(f) floats each).
+hipError_t launch_to16(int f, int prec, const float *src, uint16_t *dst, int64_t rows, hipStream_t s);
 
 }  // namespace als
