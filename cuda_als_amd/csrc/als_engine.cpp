@@ -27,6 +27,7 @@ struct DevBuf {
 
 struct Side {
     int64_t rows = 0;           // rows of the matrix this side updates
+    int64_t cols = 0;           // rows of the fixed factor matrix
     int *ptr = nullptr, *idx = nullptr;
     float *val = nullptr;
     int4 *units = nullptr, *splits = nullptr;
@@ -278,8 +279,7 @@ UpdateArgs side_args(als_engine *e, const Side &s, const float *Y, const uint16_
     a.zero32 = e->zero32;
     a.zero16 = e->zero16;
     {
-        const int64_t ny = &s == &e->side[0] ? e->n : e->m;  // rows of Y
-        const int64_t sb = ny * e->sh * (int64_t)sizeof(uint16_t), yb = ny * e->ld * (int64_t)sizeof(float);
+        const int64_t sb = s.cols * e->sh * (int64_t)sizeof(uint16_t), yb = s.cols * e->ld * (int64_t)sizeof(float);
         a.ys_bytes = sb <= INT32_MAX ? (int)sb : 0;
         a.y_bytes = yb <= INT32_MAX ? (int)yb : 0;
     }
@@ -579,8 +579,8 @@ int als_set_train(als_engine *e, int64_t m, int64_t n, int64_t nnz, const int *c
     e->n = n;
     e->nnz = nnz;
     Side &su = e->side[0], &si = e->side[1];
-    su.rows = m;
-    si.rows = n;
+    su.rows = si.cols = m;
+    si.rows = su.cols = n;
     if ((rc = dev_alloc(e, &su.ptr, m + 1)) || (rc = dev_alloc(e, &su.idx, nnz)) || (rc = dev_alloc(e, &su.val, nnz)) ||
         (rc = dev_alloc(e, &si.ptr, n + 1)) || (rc = dev_alloc(e, &si.idx, nnz)) || (rc = dev_alloc(e, &si.val, nnz)) ||
         (rc = dev_alloc(e, &e->coo_row, nnz)) ||

@@ -120,3 +120,43 @@ def test_fp32_factors_beyond_two_gib():
         e.update(ca.ALS_SIDE_USERS)
         got = e.get_factors(ca.ALS_SIDE_USERS)
     assert rel(got, want) <= 1e-4
+
+
+@pytest.mark.parametrize("side", [ca.ALS_SIDE_USERS, ca.ALS_SIDE_ITEMS])
+@pytest.mark.parametrize("shape", [(40, 1500), (1500, 40)])
+@pytest.mark.parametrize("prec", list(ORACLE_PREC))
+@pytest.mark.parametrize("f", [64, 100])
+def test_row_ranges_of_oblong_matrices(f, prec, shape, side):
+    """als_update_rows on matrices with far more columns than rows and the
+    other way round (a range's fixed side is as long as its own matrix's
+    other dimension, whichever is larger): the rows of the range equal the
+    whole half-sweep's, bit for bit, the others keep their values, and the
+    half-sweep is within 1e-4 of the oracle."""
+    from cuda_als_amd import _capi as A
+    m, n = shape
+    rng = np.random.default_rng(m + f)
+    mask = rng.random((m, n)) < 0.12
+    idx = np.nonzero(mask)[1]
+    d = ca.from_arrays(m, n, np.concatenate([[0], np.cumsum(mask.sum(1))]), idx, rng.integers(1, 6, idx.size),
+                       [0], [0], [3.0])
+    U0, V0 = ((0.4 * rng.standard_normal((r, f))).astype(np.float32) for r in (m, n))
+    rows = m if side == ca.ALS_SIDE_USERS else n
+    first, count = rows // 3, rows // 2
+    with E.Engine(E.make_config(f, 0.05, 1, E.SolveType.CHOL, prec), d) as e:
+        out = []
+        for ranged in (False, True):
+            e.set_factors(0, U0)
+            e.set_factors(1, V0)
+            if ranged:
+                assert A.lib.als_update_rows(e.h, side, first, count, 1) == 0
+            else:
+                e.update(side)
+            out.append(e.get_factors(side))
+    old = U0 if side == ca.ALS_SIDE_USERS else V0
+    inside = np.zeros(rows, bool)
+    inside[first:first + count] = True
+    assert np.array_equal(out[1][inside], out[0][inside]) and np.array_equal(out[1][~inside], old[~inside])
+    lists = (d.csr_ptr, d.csr_idx, d.csr_val, V0) if side == ca.ALS_SIDE_USERS else (d.csc_ptr, d.csc_idx, d.csc_val, U0)
+    want = O.update_rows(O.config(f, 0.05, O.SOLVE_CHOL, gram_prec=ORACLE_PREC[prec]), np.arange(rows), *lists[:3],
+                         lists[3].astype(np.float64))
+    assert rel(out[0], want) <= 1e-4
