@@ -1560,48 +1560,41 @@ __device__ __forceinline__ void store_colform(float *dst, const float (&v)[T]) {
 // are complete at the end of step J, so y[J] is formed there and only one
 // row-form partial and one row form of v are live at a time. Each partial
 // sums its terms in ascending block order.
-// v's row forms are read from vs (16T floats of this wave's LDS), one 16-byte
-// read a block behind one round of writes, and a block's row-form sums are
-// scattered over the lanes and moved by one shuffle: with four shuffles for
-// the row form and four full sums over 16 lanes a block, as before, the
-// exchanges were half of the mat-vec's instructions. One sweep at the ml10M
-// shape: f = 100 FP32 1.274 -> 1.261 ms, f = 80 with the 16-bit Gram 0.585 ->
-// 0.580 ms; 8,192 batched systems of f = 100 100.9 -> 99.8 us (waiting for
-// their matrices, and the rows for their gathers, is most of the rest).
+// (The row forms through LDS and the sums scattered over the lanes, for fewer
+// exchanges, ran the FP32 sweeps 1% faster but the batched systems with an
+// FP16 A at f = 100 in 0.264 instead of 0.176 ms: not kept.)
 template <int T, int NT>
-__device__ __forceinline__ void matvec_f32(const f32x4 (&A)[NT], int f, const float (&v)[T], float (&y)[T],
-                                           float *vs) {
-    const int l = lane(), q = l >> 4, c = l & 15;
-    store_colform<T>(vs, v);
-    wave_sync();
+__device__ __forceinline__ void matvec_f32(const f32x4 (&A)[NT], int f, const float (&v)[T], float (&y)[T]) {
+    const int c = lane() & 15;
     float pc[T];
 #pragma unroll
     for (int I = 0; I < T; ++I) pc[I] = 0.f;
 #pragma unroll
     for (int J = 0; J < T; ++J) {
-        const f32x4 vr = *reinterpret_cast<const f32x4 *>(vs + 16 * J + 4 * q);
-        f32x4 pr = A[tile_id(J, J)] * v[J];
+        const f32x4 vr = col_to_row(v[J]);
+        f32x4 pr = f32x4{0.f, 0.f, 0.f, 0.f};
+        pr += A[tile_id(J, J)] * v[J];
 #pragma unroll
         for (int I = J + 1; I < T; ++I) {
             const f32x4 t = A[tile_id(I, J)];
             pc[I] += t[0] * vr[0] + t[1] * vr[1] + t[2] * vr[2] + t[3] * vr[3];
             pr += t * v[I];
         }
-        // row 16J + c: lane (c / 4, c) holds the total for register c % 4 of row c / 4
-        const float s = rows16_scatter4(pr);
-        const float yc = __shfl(s, ((c >> 2) << 4) | c, WAVE) + q4_sum(pc[J]);
+        f32x4 s;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[r] = row16_sum(pr[r]);
+        const float yc = row_to_col(s) + q4_sum(pc[J]);
         y[J] = (16 * J + c < f) ? yc : 0.f;
     }
-    wave_sync();  // vs read before the next product's writes
 }
 
 // cuMF CG (cumf_als_cg/cg.cu:37-232) on the register tiles: warm start x,
 // `iters` iterations, exit when r.r < tol after an update; p.Ap == 0 stops.
 template <int T, int NT>
 __device__ __forceinline__ void cg_regs(const f32x4 (&A)[NT], int f, const float (&b)[T], float (&x)[T], int iters,
-                                        float tol, float *vs) {
+                                        float tol) {
     float r[T], p[T], ap[T];
-    matvec_f32<T>(A, f, x, ap, vs);
+    matvec_f32<T>(A, f, x, ap);
 #pragma unroll
     for (int J = 0; J < T; ++J) {
         r[J] = b[J] - ap[J];
@@ -1609,7 +1602,7 @@ __device__ __forceinline__ void cg_regs(const f32x4 (&A)[NT], int f, const float
     }
     float rsold = colform_dot(r, r, T);
     for (int it = 0; it < iters; ++it) {
-        matvec_f32<T>(A, f, p, ap, vs);
+        matvec_f32<T>(A, f, p, ap);
         const float pap = colform_dot(p, ap, T);
         if (pap == 0.f) break;
         const float alpha = rsold / pap;
@@ -2006,7 +1999,7 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
                             for (int r = 0; r < 4; ++r) acc[t][r] = (float)(_Float16)acc[t][r];
                     }
                     load_colform<T>(a.X + (int64_t)row * G::LD, f, x);
-                    cg_regs<T>(acc, f, bv, x, a.cg_iters, a.cg_tol, xs);
+                    cg_regs<T>(acc, f, bv, x, a.cg_iters, a.cg_tol);
                 }
                 bool finite = true;
 #pragma unroll

@@ -447,7 +447,6 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(T <= 7 ? 2
     constexpr int NT = T * (T + 1) / 2;
     const int l = lane(), q = l >> 4, c = l & 15;
     const int f = a.f;
-    __shared__ __attribute__((aligned(16))) float vs[16 * T];
     for (int sys = blockIdx.x; sys < a.batch; sys += gridDim.x) {
         const int64_t base = (int64_t)sys * f * f;
         auto at = [&](int i, int j) -> float {
@@ -522,7 +521,7 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(T <= 7 ? 2
             bc[J] = i < f ? a.b[(int64_t)sys * f + i] : 0.f;
             xc[J] = i < f ? a.x[(int64_t)sys * f + i] : 0.f;
         }
-        cg_regs<T>(acc, f, bc, xc, a.iters, a.tol, vs);
+        cg_regs<T>(acc, f, bc, xc, a.iters, a.tol);
         if (q == 0) {
 #pragma unroll
             for (int J = 0; J < T; ++J)
