@@ -6,7 +6,7 @@ one full sweep (all users from V, then all items from U) with the data
 already resident in HBM, timed as replays of the captured sweep graph. The
 mixed-precision path (FP16 Gram on MFMA with FP32 accumulation, FP32
 Cholesky, FP64-residual refinement) is the measured line; the plain FP32 path
-(FP32 MFMA Gram, FP32 Cholesky) is timed beside it for the speed ratio, and
+(FP32 Gram, FP32 Cholesky) is timed beside it for the speed ratio, and
 so is the reference's production solver, FP32 CG with 6 iterations. Each
 path's test RMSE over 10 sweeps from the reference init is compared with the
 FP64 oracle's trajectory of the same workload (tests/golden fixture).
@@ -406,7 +406,7 @@ def main() -> int:
         F = run(fp32_cfg, "fp32", "chol")
         fp32 = {"sweeps_per_s": a.steps / F["dt"], "users_ms": F["users_ms"], "items_ms": F["items_ms"],
                 "test_rmse": F["rmse"], "failures": int(F["info"].failures), "vs_oracle": F["vs_oracle"],
-                "solve": ("fp32 MFMA Gram, fp32 Cholesky, no refinement"
+                "solve": ("fp32 Gram (three bf16 parts per operand on MFMA), fp32 Cholesky, no refinement"
                           + (f"; rows under {list(F['info'].dual_limit)} ratings (users, items) through their "
                              f"n x n dual system" if F["info"].dual_max else ""))}
         cg_cfg = E.make_config(f, lam, a.steps, E.SolveType.CUMF_ALS_CG_FP32, E.Prec.FP32, cg_iters=6, cg_tol=1e-4,
@@ -414,7 +414,7 @@ def main() -> int:
         G = run(cg_cfg, "fp32-cg6", "cg6")
         cg6 = {"sweeps_per_s": a.steps / G["dt"], "users_ms": G["users_ms"], "items_ms": G["items_ms"],
                "test_rmse": G["rmse"], "failures": int(G["info"].failures), "vs_oracle": G["vs_oracle"],
-               "solve": "fp32 MFMA Gram, cuMF CG recurrence: 6 iterations, warm start, exit on r.r < 1e-4 "
+               "solve": "fp32 Gram, cuMF CG recurrence: 6 iterations, warm start, exit on r.r < 1e-4 "
                         "(the reference's production solver)"}
 
     # Dominant kernel: the slower half-sweep of the mixed path (its update kernel plus the dual
