@@ -35,6 +35,8 @@ struct Side {
     float *partial = nullptr;
     int nbatches = 0, nunits = 0, nsplits = 0;
     int64_t nslots = 0, split_len = 0, batch_work = 0;
+    int64_t own_work = 0;       // the batch_work that the scheduler chose for the whole side
+                                // (0: the configuration gave one)
     int grid = 0;                  // persistent waves of the default update kernel (variant 0),
                                    // at most the engine's grid_max (autotuned per side)
     int variant = 0;               // update kernel variant (1: one wave per SIMD, where built)
@@ -187,7 +189,8 @@ void free_schedule(als_engine *e, Side &s) {
 }
 
 // (Re)build one side's work schedule over rows [rb, re) and upload it;
-// replaces any previous one.
+// replaces any previous one. A batch_work other than the scheduler's own is
+// taken as it is.
 int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work,
                int64_t rb = 0, int64_t re = -1) {
     if (re < 0) re = rows;
@@ -199,7 +202,7 @@ int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t spl
         for (int64_t r = rb; r < re; r++) (dual && ptr[r + 1] - ptr[r] < s.dual_limit ? light : heavy).push_back((int)r);
     }
     Schedule sc = build_schedule(rows, ptr, (int)split_len, (int)batch_work, s.grid, e->prec,
-                                 dual || ranged ? &heavy : nullptr);
+                                 dual || ranged ? &heavy : nullptr, batch_work == s.own_work);
     Schedule sd;
     if (dual && !light.empty()) sd = build_schedule(rows, ptr, (int64_t)1 << 30, 0, e->dual_grid, e->prec, &light);
     static_assert(sizeof(Unit) == sizeof(int4) && sizeof(Split) == sizeof(int4), "unit layout");
@@ -616,9 +619,14 @@ int als_set_train(als_engine *e, int64_t m, int64_t n, int64_t nnz, const int *c
         e->yb_partial[sd] = nullptr;
         e->yb_nparts[sd] = 0;
     }
+    su.own_work = si.own_work = 0;
     if ((rc = build_side(e, su, m, csr_ptr, e->cfg.split_len, e->cfg.batch_work)) ||
         (rc = build_side(e, si, n, csc_ptr, e->cfg.split_len, e->cfg.batch_work)))
         return rc;
+    if (e->cfg.batch_work <= 0) {
+        su.own_work = su.batch_work;
+        si.own_work = si.batch_work;
+    }
     e->have_train = true;
     return ALS_OK;
 }

@@ -10,8 +10,9 @@ namespace als {
 int64_t row_solve_cost(int prec) { return prec == PREC_FP32 ? 96 : 1024; }
 
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
-                        const std::vector<int> *subset) {
+                        const std::vector<int> *subset, bool own_batches) {
     Schedule s;
+    own_batches = own_batches || batch_work <= 0;
     const int64_t solve = row_solve_cost(prec);
     const int64_t nrows = subset ? (int64_t)subset->size() : rows;
     auto row_at = [&](int64_t i) -> int64_t { return subset ? (int64_t)(*subset)[i] : i; };
@@ -49,13 +50,14 @@ Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t
     }
     std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) { return a.cost > b.cost; });
     s.units.reserve(items.size());
-    // Batches of about batch_work, heaviest rows first. Each batch but a wave's
-    // first costs an atomic on a counter that all waves share, some 10 ns, one
-    // after the other. Where an average batch is little more work than the GPU
-    // gets through in that time, the waves would wait for the counter: there
-    // the batches start large and shrink to batch_work, each taking half of
-    // what an even share of the work still left would be, and small ones are
-    // left for the end, to even out what the cost model got wrong. One sweep,
+    // Batches of batch_work, heaviest rows first. Each batch but a wave's first
+    // costs an atomic on a counter that all waves share, some 10 ns, one after
+    // the other. Where the size is the scheduler's own and an average batch is
+    // little more work than the GPU gets through in that time, the waves would
+    // wait for the counter: there the batches start large and shrink to
+    // batch_work, each taking half of what an even share of the work still left
+    // would be, and small ones are left for the end, to even out what the cost
+    // model got wrong. A caller's size is taken as it is. One sweep,
     // batch_work throughout -> shrinking: f = 64 FP32 at the ml10M shape (62,000
     // user batches of about 350) 1.16 -> 0.90 ms; f = 80, 16-bit Gram and CG
     // there (12,000 item batches of about 1,700) 0.70 -> 0.58 ms; a quarter of
@@ -83,7 +85,7 @@ Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t
         }
     };
     cut(false);
-    if (all < small * (int64_t)s.batch_begin.size()) cut(true);
+    if (own_batches && all < small * (int64_t)s.batch_begin.size()) cut(true);
     if (s.batch_begin.back() != (int)items.size()) s.batch_begin.push_back((int)items.size());
     return s;
 }

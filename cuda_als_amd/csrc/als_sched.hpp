@@ -9,9 +9,10 @@
 //     order (deterministic) and solves;
 //   * units are ordered by decreasing cost (longest-processing-time first),
 //     so the tail of the launch is made of the lightest rows;
-//   * consecutive units are grouped into batches of about `batch_work`
-//     rating-equivalents, where those would be small larger ones first;
-//     persistent waves take batches from a device queue.
+//   * consecutive units are grouped into batches of `batch_work`
+//     rating-equivalents or just above; where the scheduler chose that size and
+//     it is small, larger batches come first and shrink to it; persistent waves
+//     take batches from a device queue.
 #pragma once
 #include <cstdint>
 #include <vector>
@@ -37,7 +38,7 @@ struct Schedule {
     std::vector<int> batch_begin;  // batch b = units[batch_begin[b] .. batch_begin[b+1])
     int64_t nslots = 0;            // partial-Gram slots needed
     int64_t split_len = 0;
-    int64_t batch_work = 0;
+    int64_t batch_work = 0;        // size of a batch; of the smallest where they shrink
 };
 
 // Cost of a solve in rating-equivalents of Gram work for the given Gram
@@ -48,7 +49,10 @@ int64_t row_solve_cost(int prec);
 // split_len <= 0 and batch_work <= 0 select sizes from the total work and
 // the number of persistent waves (`grid`). subset (nullable): schedule only
 // these rows (ascending), e.g. the rows left after the dual system's.
+// own_batches: batch_work is a size that the scheduler chose for an earlier
+// schedule of these rows, and the batches may shrink to it as they may where
+// it is chosen here.
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
-                        const std::vector<int> *subset = nullptr);
+                        const std::vector<int> *subset = nullptr, bool own_batches = false);
 
 }  // namespace als

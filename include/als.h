@@ -76,7 +76,9 @@ typedef struct {
     int m_batches;       /* accepted for config compatibility; the engine never */
     int n_batches;       /*   materialises Gram matrices, so no batching is needed */
     int device;          /* HIP device ordinal */
-    int batch_work;      /* ratings per work-queue batch; 0 = chosen by the scheduler */
+    int batch_work;      /* ratings per work-queue batch; 0 = chosen by the scheduler, whose
+                            batches shrink from larger ones to the size it chose where
+                            that is small */
     int split_len;       /* rows with more ratings are split across waves; 0 = chosen */
     int use_graph;       /* replay each sweep from a captured hipGraph */
     int refine_warm;     /* 1: the first refinement step starts from the row's previous
@@ -185,8 +187,9 @@ int als_cg_update_x_tt_fp16(const float *A, float *x, const float *b, int batch,
 
 /* Host-only (no device needed): the work schedule the engine builds for one
  * side from its CSR row pointers: whole rows plus parts of rows longer than
- * split_len, heaviest first, cut into queue batches. units_out (nullable)
- * receives 4 ints per unit {row, kb, ke, split_id}, at most max_units.
+ * split_len, heaviest first, cut into queue batches (of batch_work; <= 0: as
+ * the scheduler chooses, and the statistics hold the size of its smallest).
+ * units_out (nullable) receives 4 ints per unit {row, kb, ke, split_id}, at most max_units.
  * No reference counterpart (the reference launches one block per row in row
  * order, als_model.cu:1891-1982). */
 typedef struct {
@@ -226,7 +229,10 @@ typedef struct {
 int als_autotune(als_engine *e, int sides, als_tune_result *out);
 /* Applies one side's schedule directly (e.g. a stored als_autotune result):
  * split length, batch size (<= 0: keep) and the refinement restage threshold
- * (< 0: keep). No reference counterpart. */
+ * (< 0: keep). Every batch has the size given, but for the one size that the
+ * scheduler chose for this side at als_set_train (als_config.batch_work = 0),
+ * which brings back the scheduler's own batches: a stored als_autotune result
+ * gives the batches that were tuned. No reference counterpart. */
 int als_set_schedule(als_engine *e, int side, int64_t split_len, int64_t batch_work, int restage_max);
 /* Update kernel variant of one side: 0 the default (two waves per SIMD for the
  * refinement solvers), 1 one wave per SIMD with the whole register file

@@ -39,6 +39,8 @@ def test_batches_against_waves(f, prec, grid, graph):
         for limit in {0, e.info().dual_max}:
             e.set_grid(ca.ALS_SIDE_USERS, grid)
             e.set_dual_limit(ca.ALS_SIDE_USERS, limit)
+            if limit == 0:
+                assert e.info().nbatches[0] == ROWS  # the batch size asked for, whatever the grid
             first = None
             for _ in range(4):
                 e.set_factors(ca.ALS_SIDE_USERS, np.zeros((ROWS, f), np.float32))
@@ -55,3 +57,39 @@ def test_batches_against_waves(f, prec, grid, graph):
             e.update(ca.ALS_SIDE_USERS)
             assert np.array_equal(e.get_factors(ca.ALS_SIDE_USERS), first)
             e.set_schedule(ca.ALS_SIDE_USERS, 0, 1)
+
+
+@pytest.mark.parametrize("batch_work", [0, 500])
+@pytest.mark.parametrize("prec", [E.Prec.FP32, E.Prec.FP16])
+def test_a_stored_tuning_gives_the_batches_that_were_tuned(prec, batch_work):
+    """als_autotune's result applied to a fresh engine in either order of the
+    calls: the same batches as on the tuned engine, also where the scheduler's
+    own (shrinking) ones were the fastest, and the same bits."""
+    rng = np.random.default_rng(9)
+    lengths = rng.integers(1, 200, 3000)
+    idx = np.concatenate([np.sort(rng.choice(500, n, replace=False)) for n in lengths])
+    d = ca.from_arrays(3000, 500, np.concatenate([[0], np.cumsum(lengths)]), idx, rng.integers(1, 6, idx.size),
+                       [0], [0], [3.0])
+    cfg = E.make_config(70, 0.05, 1, E.SolveType.CHOL, prec, batch_work=batch_work)
+    V0 = rng.standard_normal((500, 70)).astype(np.float32) * 0.3
+
+    def update(e):
+        e.set_factors(ca.ALS_SIDE_ITEMS, V0)
+        e.update(ca.ALS_SIDE_USERS)
+        return list(e.info().nbatches), e.get_factors(ca.ALS_SIDE_USERS)
+
+    with E.Engine(cfg, d) as e:
+        e.init_factors()
+        t = e.autotune()
+        want = update(e)
+    for order in (1, -1):
+        with E.Engine(cfg, d) as e:
+            for side in (0, 1):
+                calls = [lambda: e.set_schedule(side, t["split_len"][side], t["batch_work"][side]),
+                         lambda: e.set_grid(side, t["grid"][side]), lambda: e.set_dual_limit(side, t["dual_limit"][side])]
+                for c in calls[::order]:
+                    c()
+                if t["gram_gather"][side]:
+                    e.set_gram_gather(side, 1)
+            got = update(e)
+            assert got[0] == want[0] and np.array_equal(got[1], want[1])
