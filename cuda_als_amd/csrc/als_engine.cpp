@@ -201,10 +201,12 @@ int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t spl
     if (dual || ranged) {
         for (int64_t r = rb; r < re; r++) (dual && ptr[r + 1] - ptr[r] < s.dual_limit ? light : heavy).push_back((int)r);
     }
+    const bool slow = tiles(e->cfg.f) >= 8 || e->solve == SOLVE_CHOL_REFINE;
     Schedule sc = build_schedule(rows, ptr, (int)split_len, (int)batch_work, s.grid, e->prec,
-                                 dual || ranged ? &heavy : nullptr, batch_work == s.own_work);
+                                 dual || ranged ? &heavy : nullptr, batch_work == s.own_work, slow);
     Schedule sd;
-    if (dual && !light.empty()) sd = build_schedule(rows, ptr, (int64_t)1 << 30, 0, e->dual_grid, e->prec, &light);
+    if (dual && !light.empty())
+        sd = build_schedule(rows, ptr, (int64_t)1 << 30, 0, e->dual_grid, e->prec, &light, true, slow);
     static_assert(sizeof(Unit) == sizeof(int4) && sizeof(Split) == sizeof(int4), "unit layout");
     HIPCHK(e, hipStreamSynchronize(e->stream));
     free_schedule(e, s);

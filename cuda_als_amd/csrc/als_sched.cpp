@@ -10,7 +10,7 @@ namespace als {
 int64_t row_solve_cost(int prec) { return prec == PREC_FP32 ? 96 : 1024; }
 
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
-                        const std::vector<int> *subset, bool own_batches) {
+                        const std::vector<int> *subset, bool own_batches, bool slow_ratings) {
     Schedule s;
     own_batches = own_batches || batch_work <= 0;
     const int64_t solve = row_solve_cost(prec);
@@ -51,28 +51,40 @@ Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t
     std::stable_sort(items.begin(), items.end(), [](const Item &a, const Item &b) { return a.cost > b.cost; });
     s.units.reserve(items.size());
     // Batches of batch_work, heaviest rows first. Each batch but a wave's first
-    // costs an atomic on a counter that all waves share, some 10 ns, one after
+    // costs an atomic on a counter that all waves share, some 12 ns, one after
     // the other. Where the size is the scheduler's own and an average batch is
     // little more work than the GPU gets through in that time, the waves would
     // wait for the counter: there the batches start large and shrink to
     // batch_work, each taking half of what an even share of the work still left
     // would be, and small ones are left for the end, to even out what the cost
-    // model got wrong. A caller's size is taken as it is. One sweep,
-    // batch_work throughout -> shrinking: f = 64 FP32 at the ml10M shape (62,000
-    // user batches of about 350) 1.16 -> 0.90 ms; f = 80, 16-bit Gram and CG
-    // there (12,000 item batches of about 1,700) 0.70 -> 0.58 ms; a quarter of
-    // the netflix-shaped users, f = 100 FP32 (75,000 of about 450) 3.79 -> 3.56
-    // ms. At the netflix shape with the 16-bit Gram (19,000 item batches of
-    // 6,100) large first batches lose instead, 6.54 -> 6.64 ms: their rows take
-    // longer than the model says, and there is nothing to gain.
+    // model got wrong. A caller's size is taken as it is. One half-sweep of
+    // the users, even batches -> shrinking: ml10M shape, f = 64 FP32 838 -> 580
+    // us (62,600 -> 32,300 batches), f = 16 805 -> 490, f = 80 16-bit Gram and
+    // CG 437 -> 289; a quarter of the netflix-shaped users, f = 100 FP32 2.22 ->
+    // 2.02 ms. At the whole netflix shape with the 16-bit Gram (items, batches
+    // of 6,100 on average) there is nothing to gain, and large first batches
+    // lose: 6.54 -> 6.64 ms a sweep.
+    // No batch is larger than `most`, a size at which the counter is no
+    // bottleneck any more: of a larger one the model's error is all that is
+    // felt. Without it 16-bit users with two refinement steps lost what the
+    // short rows gain (f = 32 708 -> 773 us, f = 140 4.62 -> 5.20 ms; a quarter
+    // of the netflix shape, f = 48 1.72 -> 2.07). Where a rating takes about
+    // twice the model's time, at 8 and 9 blocks and with classic refinement,
+    // which reads a row's ratings again for each step, half the size is the
+    // better one: BF16 users at f = 128 656 us without a bound, 657 at the whole
+    // of it, 631 at half (even 952); CG items at f = 140 738, 737, 692 (even
+    // 690); refined 16-bit users at f = 32 773, 799, 682. At fewer blocks it is
+    // not: BF16 users at f = 80 724, 740, 776 (even 984), a quarter of the
+    // netflix shape.
     const int64_t small = prec == PREC_FP32 ? 768 : 4608;
+    const int64_t most = slow_ratings ? small : 2 * small;
     for (const Item &it : items) s.units.push_back(it.u);
     int64_t all = 0;
     for (const Item &it : items) all += it.cost;
     auto cut = [&](bool shrink) {
         s.batch_begin.assign(1, 0);
         int64_t left = all, acc = 0;
-        auto size_at = [&] { return std::max(s.batch_work, shrink ? left / (2 * waves) : 0); };
+        auto size_at = [&] { return std::max(s.batch_work, shrink ? std::min(most, left / (2 * waves)) : 0); };
         int64_t want = size_at();
         for (size_t i = 0; i < items.size(); i++) {
             acc += items[i].cost;

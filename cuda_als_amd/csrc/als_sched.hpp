@@ -51,8 +51,10 @@ int64_t row_solve_cost(int prec);
 // these rows (ascending), e.g. the rows left after the dual system's.
 // own_batches: batch_work is a size that the scheduler chose for an earlier
 // schedule of these rows, and the batches may shrink to it as they may where
-// it is chosen here.
+// it is chosen here. slow_ratings: a rating takes well over the model's time
+// (8 or 9 blocks, classic refinement).
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
-                        const std::vector<int> *subset = nullptr, bool own_batches = false);
+                        const std::vector<int> *subset = nullptr, bool own_batches = false,
+                        bool slow_ratings = false);
 
 }  // namespace als

@@ -33,8 +33,9 @@ def batches(tmp_path_factory):
     r = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-3000:]
 
-    def run(sizes, batch_work, grid, prec, own=False):
-        out = subprocess.run([str(exe), "1000000000", str(batch_work), str(grid), str(prec), str(int(own))],
+    def run(sizes, batch_work, grid, prec, own=False, slow=False):
+        out = subprocess.run([str(exe), "1000000000", str(batch_work), str(grid), str(prec), str(int(own)),
+                              str(int(slow))],
                              input=" ".join(map(str, sizes)), capture_output=True, text=True, timeout=60, check=True)
         work, *begin = map(int, out.stdout.split())
         begin = np.array(begin)
@@ -90,3 +91,17 @@ def test_small_batches_shrink_from_large_ones(batches):
     assert np.array_equal(batches(sizes, work, waves, A.ALS_PREC_FP32, own=True)[1], begin)
     _, begin, _ = batches(np.full(4000, 6000), 0, 64, A.ALS_PREC_FP16)
     assert np.unique(np.diff(begin)[:-1]).size == 1
+
+
+@pytest.mark.parametrize("slow", [False, True])
+@pytest.mark.parametrize("prec,most", [(A.ALS_PREC_FP32, 1536), (A.ALS_PREC_FP16, 9216)])
+def test_shrinking_batches_are_bounded(prec, most, slow, batches):
+    """However few the waves, no shrinking batch is larger than what the
+    counter asks for (half of that where ratings are slow) by more than its
+    last row."""
+    sizes = np.random.default_rng(2).poisson(120, 100000)
+    work, begin, cost = batches(sizes, 0, 3072, prec, slow=slow)
+    total = np.add.reduceat(cost, begin[:-1])
+    bound = most // (1 + slow)
+    assert bound <= total.max() < bound + cost.max() and work < bound
+    assert total[-2] < work + cost.max()
