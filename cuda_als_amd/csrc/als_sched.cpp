@@ -7,6 +7,8 @@
 
 namespace als {
 
+constexpr int64_t GPU_SIMDS = 1024;  // 256 CUs of four
+
 int64_t row_solve_cost(int prec) { return prec == PREC_FP32 ? 96 : 1024; }
 
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
@@ -23,8 +25,14 @@ Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t
     }
     const int64_t waves = std::max<int64_t>(1, grid);
     // Parts small enough that the heaviest row spreads over many waves, large
-    // enough that the partial-tile traffic stays small next to the gathers.
-    s.split_len = split_len > 0 ? split_len : std::max<int64_t>(2048, total / (waves * 8));
+    // enough that the traffic of the partial tiles stays small next to the
+    // gathers: an eighth of what each SIMD gets, however many waves of the
+    // kernel at hand fit on it (their gathers share its time). Counted by waves
+    // instead, kernels of fewer blocks, which fit more often, cut rows shorter:
+    // 16-bit Gram and CG, items of a quarter of the netflix shape, f = 80 at
+    // three waves a SIMD, parts of 2,048 653 us, of 4,322 500; f = 112 at two,
+    // 742 and 555.
+    s.split_len = split_len > 0 ? split_len : std::max<int64_t>(2048, total / (std::min(waves, GPU_SIMDS) * 8));
     s.batch_work = batch_work > 0 ? batch_work : std::max<int64_t>(solve, total / (waves * 16));
 
     struct Item { Unit u; int64_t cost; };

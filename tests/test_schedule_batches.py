@@ -105,3 +105,12 @@ def test_shrinking_batches_are_bounded(prec, most, slow, batches):
     bound = most // (1 + slow)
     assert bound <= total.max() < bound + cost.max() and work < bound
     assert total[-2] < work + cost.max()
+
+
+@pytest.mark.parametrize("prec", [A.ALS_PREC_FP32, A.ALS_PREC_FP16])
+def test_split_length_does_not_fall_with_occupancy(prec):
+    """The parts of long rows are no shorter where more waves fit on a SIMD:
+    their number is a matter of the GPU's size and the work."""
+    sizes = np.concatenate([np.full(20, 200000), np.full(9000, 3000)])
+    lens = [preview(sizes, 0, 0, grid, prec)[1].split_len for grid in (1024, 2048, 3072, 8192)]
+    assert len(set(lens)) == 1 and lens[0] > 2048 and preview(sizes, 0, 0, 256, prec)[1].split_len > lens[0]
