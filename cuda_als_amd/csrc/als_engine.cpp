@@ -502,6 +502,13 @@ int als_create(const als_config *cfg, als_engine **out) {
         int pc1 = 0;
         if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&pc1, k1, 64, e->lds) == hipSuccess && pc1 > 0)
             e->grid_v1 = pc1 * e->num_cu;
+        // From 8 blocks on (f >= 112) an FP32 Gram and its operands' parts do not
+        // fit the registers of two waves: 90 (f = 127) and 406 (f = 143) of them
+        // spill, and one wave without a spill is faster. Users and items of the
+        // ml10M shape, two waves -> one: f = 112 1.21, 1.01 -> 0.99, 0.84 ms; f = 128
+        // 1.63, 1.46 -> 1.20, 1.03; f = 143 2.62, 2.59 -> 1.81, 1.35. Below it is
+        // slower: f = 100 0.99, 0.62 -> 1.01, 0.86.
+        if (e->grid_v1 > 0 && e->prec == PREC_FP32 && e->T >= 8) e->side[0].variant = e->side[1].variant = 1;
     }
     const void *dk = dual_kernel_ptr(cfg->f, e->prec, e->solve);
     if (!rc && dk) {

@@ -145,9 +145,9 @@ struct RmseArgs {
 
 // Launchers (als_kernels_*.hip). Each returns the hipError_t of the launch.
 int update_lds_bytes(int f, int prec, int solve);
-// variant 0: the default kernel of the solver (two waves per SIMD for the
-// refinement solvers); variant 1: one wave per SIMD (warm-started refinement,
-// f >= 96; null elsewhere).
+// variant 0: the solver's usual kernel (two waves per SIMD for the refinement
+// solvers); variant 1: one wave per SIMD (warm-started refinement, f >= 96;
+// null elsewhere).
 hipError_t launch_update(int f, int prec, int solve, int variant, const UpdateArgs &a, int grid, int lds_bytes,
                          hipStream_t s);
 const void *update_kernel_ptr(int f, int prec, int solve, int variant = 0);

@@ -216,9 +216,9 @@ typedef struct {
     int restage_max[2];                  /* refinement: rows up to this long restage their
                                             ratings for the residual, longer ones keep a
                                             copy of the tiles (tuned with refine_steps > 0) */
-    int kernel_variant[2];               /* update kernel variant chosen (0: default, 1: one
+    int kernel_variant[2];               /* update kernel variant chosen (0: two waves, 1: one
                                             wave per SIMD; tried where it is built) */
-    int grid[2];                         /* persistent waves of the default update kernel
+    int grid[2];                         /* persistent waves of the variant-0 kernel
                                             chosen (the occupancy limit or down to half of
                                             it, in steps of one wave per CU; als_set_grid) */
     int dual_limit[2];                   /* rating count below which rows take the dual
@@ -234,12 +234,13 @@ int als_autotune(als_engine *e, int sides, als_tune_result *out);
  * which brings back the scheduler's own batches: a stored als_autotune result
  * gives the batches that were tuned. No reference counterpart. */
 int als_set_schedule(als_engine *e, int side, int64_t split_len, int64_t batch_work, int restage_max);
-/* Update kernel variant of one side: 0 the default (two waves per SIMD for the
- * refinement solvers), 1 one wave per SIMD with the whole register file
- * (warm-started refinement at 7 to 9 tiles; ALS_E_UNSUPPORTED elsewhere). The
- * results are identical; als_autotune times both. No reference counterpart. */
+/* Update kernel variant of one side: 0 two waves per SIMD for the refinement
+ * solvers, 1 one wave per SIMD with the whole register file (warm-started
+ * refinement at 7 to 9 tiles; ALS_E_UNSUPPORTED elsewhere). An engine starts
+ * on 0, but on 1 with an FP32 Gram at 8 and 9 tiles. The results are
+ * identical; als_autotune times both. No reference counterpart. */
 int als_set_kernel_variant(als_engine *e, int side, int variant);
-/* Persistent waves of one side's default update kernel, 1 .. als_info.grid's
+/* Persistent waves of one side's variant-0 update kernel, 1 .. als_info.grid's
  * value at als_create (the occupancy limit); the schedule is rebuilt for
  * them. Results are identical for every grid. No reference counterpart. */
 int als_set_grid(als_engine *e, int side, int grid);

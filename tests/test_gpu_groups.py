@@ -121,6 +121,28 @@ def test_one_wave_kernel_variant_equals_default(f):
     assert err.max() <= 5e-5
 
 
+@pytest.mark.parametrize("f,default", [(100, 0), (111, 0), (112, 1), (128, 1), (143, 1)])
+def test_default_variant_of_wide_fp32_systems(f, default):
+    """FP32 warm-started systems of 8 and 9 tiles (f >= 112) start on the
+    one-wave variant, the others on the two-wave one; either can be chosen
+    and both give the same bits, whole and split rows."""
+    d = ca.scaled(ca.netflix_shape(), 0.01).generate()
+    out = []
+    for variant in (None, 1 - default, default):
+        cfg = E.make_config(f, 0.05, 1, E.SolveType.CHOL, E.Prec.FP32, refine=1, refine_warm=True, split_len=500)
+        with E.Engine(cfg, d) as e:
+            for side in (0, 1):
+                if variant is not None:
+                    e.set_kernel_variant(side, variant)
+            e.init_factors()
+            e.sweep()
+            out.append((e.get_factors(0), e.get_factors(1)))
+            info = e.info()
+        assert list(info.kernel_variant) == [default if variant is None else variant] * 2
+        assert info.failures == 0 and info.nsplit_rows[1] > 0
+    assert all(np.array_equal(a, b) for other in out[1:] for a, b in zip(out[0], other))
+
+
 @pytest.mark.parametrize("f,prec", [(100, E.Prec.FP16), (97, E.Prec.BF16), (120, E.Prec.FP16), (128, E.Prec.FP16)])
 def test_one_wave_register_gathers_equal_default(f, prec):
     """The one-wave variant with the register-gather Gram (the Gram the
