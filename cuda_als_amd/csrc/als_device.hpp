@@ -799,8 +799,9 @@ __device__ __forceinline__ void gram_row32(const UpdateArgs &a, int64_t rs, int 
 
 // The Gram of ratings rs .. rs + n - 1 of a row; with AUG = false also b, in
 // column form, each lane row q holding its share of the ratings (q4_sum adds
-// them). With AUG, b is row f of the tiles.
-template <int T, int E, bool AUG>
+// them). With AUG, b is row f of the tiles. PIPE32: on the FP32 matrix pipe,
+// for the kernels whose registers gram_row32 would overflow.
+template <int T, int E, bool AUG, bool PIPE32>
 __device__ __forceinline__ void gram_row(const UpdateArgs &a, int64_t rs, int n, f32x4 (&acc)[T * (T + 1) / 2],
                                          float (&bc)[T], char *lds) {
     using G = Geo<T, E, AUG>;
@@ -821,9 +822,31 @@ __device__ __forceinline__ void gram_row(const UpdateArgs &a, int64_t rs, int n,
         gram_row16_piped<T, E, AUG>(a, rs, n, acc, bc, lds);
         return;
     }
-    if constexpr (E == PREC_FP32) {
+    if constexpr (E == PREC_FP32 && !PIPE32) {
         gram_row32<T, AUG>(a, rs, n, acc, bc, lds);
         return;
+    }
+    if constexpr (PIPE32) {
+        static_assert(E == PREC_FP32 && AUG);
+        const float *Ys = reinterpret_cast<const float *>(stage);
+        const int q = l >> 4, c = l & 15;
+        for (int k0 = 0; k0 < n; k0 += CHUNK) {
+            stage_chunk<T, E, AUG>(a, rs, k0, min(CHUNK, n - k0), lds);
+#pragma unroll
+            for (int ks = 0; ks < CHUNK / 4; ++ks) {
+                float F[T];
+#pragma unroll
+                for (int I = 0; I < T; ++I) F[I] = Ys[(4 * ks + q) * G::YR + 16 * I + c];
+                F[T - 1] = c <= (a.f & 15) ? F[T - 1] : 0.f;  // no chunk writes the columns past f
+#pragma unroll
+                for (int I = 0; I < T; ++I)
+#pragma unroll
+                    for (int J = 0; J <= I; ++J)
+                        acc[tile_id(I, J)] =
+                            __builtin_amdgcn_mfma_f32_16x16x4f32(F[J], F[I], acc[tile_id(I, J)], 0, 0, 0);
+            }
+            wave_sync();
+        }
     }
     if constexpr (E != PREC_FP32 && T > 8) {
         stage_clear<T, E, AUG>(a.f, stage);
@@ -1871,7 +1894,14 @@ __device__ __forceinline__ void run_batch(const UpdateArgs &a, int b, char *lds)
             }
             if (n > 0) {
                 float bv[T];  // b, column form (AUG = false)
-                gram_row<T, E, AUG>(a, w.y, w.z - w.y, acc, bv, lds);
+                // Classic refinement of 9 blocks keeps two waves per SIMD (its residual
+                // hides nothing else), and the three-part operands beside 45 tiles
+                // spill 601 registers there against the FP32 pipe's 292: f = 143, users
+                // and items of the ml10M shape 6.20, 2.96 -> 6.01, 2.93 ms, of a quarter
+                // of the netflix shape 13.5, 7.04 -> 13.1, 6.87. At 8 blocks (221
+                // spilt) the parts are still faster: f = 120 4.66, 2.36 -> 4.10, 2.01 ms.
+                constexpr bool PIPE32 = E == PREC_FP32 && T == 9 && S == SOLVE_CHOL_REFINE;
+                gram_row<T, E, AUG, PIPE32>(a, w.y, w.z - w.y, acc, bv, lds);
                 if constexpr (!AUG) {
 #pragma unroll
                     for (int J = 0; J < T; ++J) bv[J] = q4_sum(bv[J]);
