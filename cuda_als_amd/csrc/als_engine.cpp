@@ -885,12 +885,10 @@ int als_save_libmf(als_engine *e, const char *path) {
 
 namespace {
 
-// Bytes of the saved factorisation of one side: the tiles of the augmented
-// system, 256 floats each, per row (at f = 16T, where the systems are one
-// block smaller, less of it is used).
+// Bytes of the saved factorisation of one side: each row's tiles.
 int64_t factor_save_bytes(const als_engine *e, int sd) {
     const int64_t rows = sd == 0 ? e->m : e->n;
-    return std::max<int64_t>(1, rows) * (int64_t)(e->T * (e->T + 1) / 2) * 256 * (int64_t)sizeof(float);
+    return std::max<int64_t>(1, rows) * factor_floats(e->cfg.f) * (int64_t)sizeof(float);
 }
 
 int forward_impl(als_engine *e, int sd, const float *d_Y, float *d_X, const float *d_lambda_rows, float *Ls) {
@@ -944,7 +942,7 @@ int adjoint_impl(als_engine *e, int sd, const float *d_Y, const float *d_X, cons
             float *dpartial = nullptr;
             int rc = dev_alloc(e, &dparts, parts.size());
             if (!rc) rc = dev_alloc(e, &dcolpart, colpart.size());
-            if (!rc) rc = dev_alloc(e, &dpartial, std::max<size_t>(1, parts.size()) * e->ld);
+            if (!rc) rc = dev_alloc(e, &dpartial, std::max<size_t>(1, parts.size()) * 16 * tiles(e->cfg.f));
             hipError_t st = hipSuccess;
             if (!rc && !parts.empty())
                 st = hipMemcpyAsync(dparts, parts.data(), parts.size() * sizeof(int4), hipMemcpyHostToDevice,

@@ -129,7 +129,7 @@ struct YbarArgs {
     // colpart[c] .. colpart[c+1]-1, in order; partial: one row per part
     const int4 *parts;
     const int *colpart;
-    float *partial;             // nparts x row_stride(f)
+    float *partial;             // nparts x 16 tiles(f)
     int nparts;
 };
 constexpr int YBAR_PART = 1024;

@@ -94,6 +94,46 @@ def test_padding_of_caller_buffers(f, prec):
             assert not t[:, f:].any() and t[:, :f].any()
 
 
+@pytest.mark.parametrize("f", [1, 16, 17, 48, 64, 100, 128, 143])
+def test_saved_factors_fill_what_they_ask_for(f):
+    """als_factor_save_bytes is what the forward pass stores, the tiles of the
+    f x f system for every row that has ratings, to the last of them: nothing
+    is written past it, and the adjoint from a buffer of just that size equals
+    the one from the engine's own."""
+    import torch
+    d, _, V0 = matrix(f)
+    with E.Engine(E.make_config(f, 0.05, 1, E.SolveType.CHOL, E.Prec.FP32), d) as e:
+        ld, T = e.info().ld, (f + 15) // 16
+        row = T * (T + 1) // 2 * 1024
+        nbytes = e.factor_save_bytes(ca.ALS_SIDE_USERS)
+        assert nbytes == d.m * row and e.factor_save_bytes(ca.ALS_SIDE_ITEMS) == d.n * row
+        e.set_stream(torch.cuda.Stream().cuda_stream)
+        save = torch.full((nbytes // 4 + 4096,), 7.0, device="cuda")
+        Y = torch.zeros(d.n, ld, device="cuda")
+        Y[:, :f] = torch.tensor(V0, device="cuda")
+        g = torch.zeros(d.m, ld, device="cuda")
+        g[:, :f] = 1e-2
+        out = []
+        for own in (False, True):
+            X, xbar, ybar = (torch.empty(r, ld, device="cuda") for r in (d.m, d.m, d.n))
+            lbar = torch.empty(d.m, device="cuda")
+            torch.cuda.synchronize()
+            if own:
+                e.forward_dev(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), None)
+                e.adjoint_dev(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), g.data_ptr(), xbar.data_ptr(),
+                              lbar.data_ptr(), ybar.data_ptr())
+            else:
+                e.forward_dev_ws(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), None, save.data_ptr(), nbytes)
+                e.adjoint_dev_ws(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), save.data_ptr(), nbytes, g.data_ptr(),
+                                 xbar.data_ptr(), lbar.data_ptr(), ybar.data_ptr())
+            torch.cuda.synchronize()
+            out.append((X, xbar, ybar, lbar))
+        with pytest.raises(ca.AlsError):
+            e.forward_dev_ws(ca.ALS_SIDE_USERS, Y.data_ptr(), X.data_ptr(), None, save.data_ptr(), nbytes - 4)
+    assert (save[nbytes // 4:] == 7.0).all() and (save[:nbytes // 4].view(d.m, row // 4)[1:, -256:] != 7.0).any(1).all()
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 def test_fp32_factors_beyond_two_gib():
     """A fixed side past 2 GiB takes the FP32 Gram's 64-bit addresses instead
     of buffer offsets: users whose items lie at both ends of it, against the
