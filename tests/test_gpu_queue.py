@@ -15,12 +15,12 @@ pytestmark = pytest.mark.gpu
 ROWS, COLS, PER_ROW = 96, 40, 9
 
 
-def matrix():
+def matrix(rows=ROWS):
     """Every user has PER_ROW ratings, so a batch of work 1 is one row."""
     rng = np.random.default_rng(5)
-    idx = np.concatenate([np.sort(rng.choice(COLS, PER_ROW, replace=False)) for _ in range(ROWS)])
+    idx = np.sort(rng.random((rows, COLS)).argsort(1)[:, :PER_ROW], 1).ravel()
     val = rng.integers(1, 6, idx.size)
-    return ca.from_arrays(ROWS, COLS, np.arange(ROWS + 1) * PER_ROW, idx, val, [0], [0], [3.0])
+    return ca.from_arrays(rows, COLS, np.arange(rows + 1) * PER_ROW, idx, val, [0], [0], [3.0])
 
 
 @pytest.mark.parametrize("graph", [False, True])
@@ -28,7 +28,8 @@ def matrix():
 @pytest.mark.parametrize("f,prec", [(16, E.Prec.FP32), (70, E.Prec.FP16)])
 def test_batches_against_waves(f, prec, grid, graph):
     """f = 70 sends every row here through the dual kernel unless its limit is
-    0; both are run. FP32 factors within 1e-4 of the oracle on the exact
+    0; both are run (the dual kernel's waves are not the grid's: its own
+    boundary is below). FP32 factors within 1e-4 of the oracle on the exact
     factors (as elsewhere for one half-sweep), FP16 within 1e-4 on the
     rounded ones."""
     d = matrix()
@@ -93,3 +94,34 @@ def test_a_stored_tuning_gives_the_batches_that_were_tuned(prec, batch_work):
                     e.set_gram_gather(side, 1)
             got = update(e)
             assert got[0] == want[0] and np.array_equal(got[1], want[1])
+
+
+@pytest.mark.parametrize("graph", [False, True])
+@pytest.mark.parametrize("prec", [E.Prec.FP32, E.Prec.FP16])
+@pytest.mark.parametrize("rows", [-1, 0, 1, 2000, 30000])
+def test_dual_batches_against_waves(rows, prec, graph):
+    """The dual kernel's tickets: as many one-row batches as its waves (four a
+    SIMD, 16 a CU), one fewer, one more and 2,000 more, and 30,000 rows in
+    batches that shrink; the same bits from launch to launch, directly and
+    from a graph, and within 1e-4 of the oracle."""
+    import torch
+    waves = 16 * torch.cuda.get_device_properties(0).multi_processor_count
+    rows = rows if rows == 30000 else waves + rows
+    d = matrix(rows)
+    V0 = np.random.default_rng(1).standard_normal((COLS, 70)).astype(np.float32) * 0.3
+    want = O.update_rows(O.config(70, 0.05, O.SOLVE_CHOL, gram_prec=O.PREC_FP16 if prec == E.Prec.FP16 else O.PREC_EXACT),
+                         np.arange(rows), d.csr_ptr, d.csr_idx, d.csr_val, V0.astype(np.float64))
+    with E.Engine(E.make_config(70, 0.05, 1, E.SolveType.CHOL, prec, use_graph=graph), d) as e:
+        info = e.info()
+        assert info.dual_rows[0] == rows
+        assert info.nbatches[0] == rows if rows < 30000 else waves < info.nbatches[0] < rows
+        first = None
+        for _ in range(4):
+            e.set_factors(ca.ALS_SIDE_USERS, np.zeros((rows, 70), np.float32))
+            e.set_factors(ca.ALS_SIDE_ITEMS, V0)
+            (e.sweep if graph else lambda: e.update(ca.ALS_SIDE_USERS))()
+            U = e.get_factors(ca.ALS_SIDE_USERS)
+            first = U if first is None else first
+            assert np.array_equal(U, first)
+        err = np.abs(first - want).max(axis=1) / np.maximum(1.0, np.abs(want).max(axis=1))
+        assert e.info().failures == 0 and err.max() <= 1e-4, err.max()
