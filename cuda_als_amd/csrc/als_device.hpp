@@ -136,9 +136,10 @@ template <int T, int E, bool AUG = true> struct Geo {
     static constexpr int DUAL_TD = TA >= 5 ? (TA - 2 < ALS_DUAL_TD_MAX ? TA - 2 : ALS_DUAL_TD_MAX) : 0;
     // The double-buffered LDS-DMA Gram (gram_row16_dma): two rating-major
     // buffers of CHUNK x FP halves, then a second ibuf/rbuf pair (256 bytes).
-    // A chunk's tasks must fit a wave (T <= 8). Where T % 4 == 0 the stage's
-    // 32-byte column blocks are permuted by row (gram_dma_loop) to keep a
-    // transposing read's four rows on distinct LDS banks.
+    // A chunk's tasks must fit a wave (T <= 8). Where T % 4 == 0 (f = 64 of the
+    // ranks it is built for) the stage's 32-byte column blocks are permuted by
+    // row (gram_dma_loop) to keep a transposing read's four rows on distinct
+    // LDS banks.
     static constexpr bool DMA_GRAM = gram_dma_built(TA, E);
     static constexpr int DMA_STAGE_BYTES = 2 * CHUNK * FP * 2 + 256;
     static constexpr int GRAM_STAGE_BYTES =
@@ -436,7 +437,8 @@ __device__ __forceinline__ void gram_row16_piped(const UpdateArgs &a, int64_t rs
 // T % 4 == 0: a stage row is a multiple of 128 bytes, and the four rows of a
 // transposing read would share LDS banks; column block I of row k is kept at
 // block I ^ (k % 4) instead (the lane that fills a slot loads that slot's
-// column, the operand reads of block I take I ^ (their row % 4)).
+// column, the operand reads of block I take I ^ (their row % 4)). Of f = 16T
+// only: the rating column of an augmented system is written unpermuted.
 template <int T, int E, bool AUG>
 __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, int n,
                                               f32x4 (&acc)[T * (T + 1) / 2], float (&bc)[T],
@@ -453,6 +455,7 @@ __device__ __forceinline__ void gram_dma_loop(const UpdateArgs &a, int64_t rs, i
     const int f = a.f;
     const bool active = l < 4 * NS;
     constexpr bool SWZ = T % 4 == 0;
+    static_assert(!(AUG && SWZ), "the rating column is not permuted");
     const int g = l / NS, s = l - g * NS;
     const int soff2 = 16 * (SWZ ? s ^ (2 * (g & 3)) : s);  // row 4e + g of the chunk: row % 4 = g % 4
     const int rrow = (8 * (l >> 4) + ((l & 15) >> 2)) * RS + 4 * (l & 3);
@@ -652,11 +655,13 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u32x4 &a, const u32x4 &b, const
 // (T % 4 == 0) or (k / 2) % 2, which puts them 16 banks apart too.
 // Against the FP32 pipe's form (a chunk gathered through registers, then
 // 16x16x4 MFMAs, nothing in flight meanwhile), one sweep: f = 100 on a quarter
-// of the netflix-shaped users (24.8M ratings) 7.02 -> 3.37 ms; at the ml10M
-// shape f = 100 with CG 3.50 -> 1.23 ms, f = 64 1.50 -> 0.99 ms. The solutions'
-// error against 64 bits fell (1.6e-5 -> 7.9e-6 on the first: the 16x16x32 form
-// rounds its sums less often). At f = 100 the splits issue about 310 VALU
-// instructions and the tiles 168 MFMAs (2,688 busy cycles) a chunk.
+// of the netflix-shaped users (24.8M ratings) 7.06 -> 3.48 ms; at the ml10M
+// shape f = 100 with CG 3.50 -> 1.29 ms, f = 64 1.50 -> 0.98 ms. The solutions'
+// error against 64 bits fell (1.6e-5 -> 4.1e-6 on the first), for the chunks'
+// sums are rounded to nearest. At f = 100 the splits issue about 310 VALU
+// instructions and the tiles 168 MFMAs (2,688 busy cycles) a chunk. The parts
+// of values below 2^-109 underflow and leave fewer bits of them (their squares
+// are below FP32's range all the same).
 template <int T, bool AUG>
 __device__ __forceinline__ void gram_row32(const UpdateArgs &a, int64_t rs, int n, f32x4 (&acc)[T * (T + 1) / 2],
                                            float (&bc)[T], char *lds) {

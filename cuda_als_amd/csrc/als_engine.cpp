@@ -494,7 +494,9 @@ int als_create(const als_config *cfg, als_engine **out) {
         per_cu = std::max(1, per_cu);
         e->side[0].grid = e->side[1].grid = e->grid_max = per_cu * e->num_cu;
         // restaging a row moves 2 FP bytes per rating; a round trip of the
-        // tile copy 2 NT KiB: equal at 32 (T + 1) ratings
+        // tile copy 2 NT KiB: equal at 32 (T + 1) ratings of an augmented
+        // system (f = 16T copies a block less and breaks even 32 ratings
+        // earlier, but keeps its residuals where callers had them)
         e->side[0].restage_max = e->side[1].restage_max = 32 * (e->T + 1);
     }
     if (const void *k1 = rc ? nullptr : update_kernel_ptr(cfg->f, e->prec, e->solve, 1)) {

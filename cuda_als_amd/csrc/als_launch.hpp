@@ -81,11 +81,12 @@ struct UpdateArgs {
 
 // Augmented tile counts (als_info.T) and precisions whose update kernels carry
 // the LDS-DMA Gram: a 16-bit Gram, at most 8 tiles (a chunk's gather tasks fit
-// a wave) and T % 4 != 0.
+// a wave) and T % 4 != 0 (the rating column of an augmented system would need
+// the banks' permutation of gram_dma_loop). f = 48, 112 and 128 go by the same
+// count, though their kernels of one block fewer would meet these conditions:
+// they gather through registers.
 constexpr bool gram_dma_built(int T, int prec) { return prec != PREC_FP32 && T <= 8 && T % 4 != 0; }
 
-// Several models (different f) on one rating matrix, one launch: batch b of
-// the combined queue is batch b - first[k] of model k (first[k] <= b < first[k+1]).
 constexpr int MAX_MODELS = 4;  // engines per group (als_group_*)
 
 struct AdjointArgs {
