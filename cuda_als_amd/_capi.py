@@ -26,6 +26,7 @@ ALS_PREC_FP32, ALS_PREC_BF16, ALS_PREC_FP16 = 0, 1, 2
 ALS_SIDE_USERS, ALS_SIDE_ITEMS = 0, 1
 ALS_RMSE_TEST, ALS_RMSE_TRAIN = 0, 1
 ALS_INIT_REFERENCE, ALS_INIT_ZERO = 0, 1
+ALS_BATCH_SHRINKS = 1 << 40
 ALS_SYNTH_UNIFORM_PAIRS, ALS_SYNTH_LOGNORMAL_ROWS = 0, 1
 
 STATUS_NAMES = {0: "ALS_OK", -1: "ALS_E_INVALID", -2: "ALS_E_HIP", -3: "ALS_E_IO", -4: "ALS_E_STATE",

@@ -35,8 +35,8 @@ struct Side {
     float *partial = nullptr;
     int nbatches = 0, nunits = 0, nsplits = 0;
     int64_t nslots = 0, split_len = 0, batch_work = 0;
-    int64_t own_work = 0;       // the batch_work that the scheduler chose for the whole side
-                                // (0: the configuration gave one)
+    bool shrinks = true;        // batches may shrink to batch_work (als_sched.cpp); false: all of that size
+    bool shrunk = false;        // and do in the present schedule
     int grid = 0;                  // persistent waves of the default update kernel (variant 0),
                                    // at most the engine's grid_max (autotuned per side)
     int variant = 0;               // update kernel variant (1: one wave per SIMD, where built)
@@ -189,8 +189,7 @@ void free_schedule(als_engine *e, Side &s) {
 }
 
 // (Re)build one side's work schedule over rows [rb, re) and upload it;
-// replaces any previous one. A batch_work other than the scheduler's own is
-// taken as it is.
+// replaces any previous one.
 int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work,
                int64_t rb = 0, int64_t re = -1) {
     if (re < 0) re = rows;
@@ -203,7 +202,7 @@ int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t spl
     }
     const bool slow = tiles(e->cfg.f) >= 8 || e->solve == SOLVE_CHOL_REFINE;
     Schedule sc = build_schedule(rows, ptr, (int)split_len, (int)batch_work, s.grid, e->prec,
-                                 dual || ranged ? &heavy : nullptr, batch_work == s.own_work, slow);
+                                 dual || ranged ? &heavy : nullptr, s.shrinks, slow);
     Schedule sd;
     if (dual && !light.empty())
         sd = build_schedule(rows, ptr, (int64_t)1 << 30, 0, e->dual_grid, e->prec, &light, true, slow);
@@ -238,6 +237,7 @@ int build_side(als_engine *e, Side &s, int64_t rows, const int *ptr, int64_t spl
     s.nslots = sc.nslots;
     s.split_len = sc.split_len;
     s.batch_work = sc.batch_work;
+    s.shrunk = sc.shrunk;
     HIPCHK(e, hipStreamSynchronize(e->stream));
     return ALS_OK;
 }
@@ -630,14 +630,10 @@ int als_set_train(als_engine *e, int64_t m, int64_t n, int64_t nnz, const int *c
         e->yb_partial[sd] = nullptr;
         e->yb_nparts[sd] = 0;
     }
-    su.own_work = si.own_work = 0;
+    su.shrinks = si.shrinks = e->cfg.batch_work <= 0;
     if ((rc = build_side(e, su, m, csr_ptr, e->cfg.split_len, e->cfg.batch_work)) ||
         (rc = build_side(e, si, n, csc_ptr, e->cfg.split_len, e->cfg.batch_work)))
         return rc;
-    if (e->cfg.batch_work <= 0) {
-        su.own_work = su.batch_work;
-        si.own_work = si.batch_work;
-    }
     e->have_train = true;
     return ALS_OK;
 }
@@ -1054,6 +1050,9 @@ int als_adjoint_dev_ws(als_engine *e, int sd, const float *d_Y, const float *d_X
 
 // Applies a schedule directly (a result of als_autotune, say); values <= 0
 // keep the current ones.
+// A side's batch size as als_set_schedule takes it to give the same batches.
+static int64_t reported_work(const Side &s) { return s.batch_work | (s.shrunk ? ALS_BATCH_SHRINKS : 0); }
+
 extern "C" int als_set_schedule(als_engine *e, int sd, int64_t split_len, int64_t batch_work, int restage_max) {
     if (!e) return ALS_E_INVALID;
     if (!e->have_train) return set_err(e, ALS_E_STATE, "set the train data first");
@@ -1061,9 +1060,12 @@ extern "C" int als_set_schedule(als_engine *e, int sd, int64_t split_len, int64_
     Side &s = e->side[sd];
     drop_graph(e);
     if (restage_max >= 0) s.restage_max = restage_max;
+    if (batch_work > 0) {
+        s.shrinks = (batch_work & ALS_BATCH_SHRINKS) != 0;
+        s.batch_work = batch_work & ~ALS_BATCH_SHRINKS;
+    }
     if (split_len > 0 || batch_work > 0)
-        return build_side(e, s, s.rows, e->hptr[sd].data(), split_len > 0 ? split_len : s.split_len,
-                          batch_work > 0 ? batch_work : s.batch_work);
+        return build_side(e, s, s.rows, e->hptr[sd].data(), split_len > 0 ? split_len : s.split_len, s.batch_work);
     return ALS_OK;
 }
 
@@ -1147,7 +1149,7 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
         Side &s = e->side[sd];
         if (!(sides & (1 << sd)) || s.rows == 0) {
             res.split_len[sd] = s.split_len;
-            res.batch_work[sd] = s.batch_work;
+            res.batch_work[sd] = reported_work(s);
             res.restage_max[sd] = s.restage_max;
             res.kernel_variant[sd] = s.variant;
             res.grid[sd] = s.grid;
@@ -1321,7 +1323,7 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
         res.best_ms[sd] = best;
         res.candidates[sd] = (int)cand.size();
         res.split_len[sd] = s.split_len;
-        res.batch_work[sd] = s.batch_work;
+        res.batch_work[sd] = reported_work(s);
     }
     (void)hipEventDestroy(ev[0]);
     (void)hipEventDestroy(ev[1]);
@@ -1542,7 +1544,7 @@ extern "C" int als_schedule_preview(int64_t rows, const int *ptr, int split_len,
         return ALS_E_INVALID;
     for (int64_t r = 0; r < rows; r++)
         if (ptr[r + 1] < ptr[r]) return ALS_E_INVALID;
-    Schedule sc = build_schedule(rows, ptr, split_len, batch_work, grid, gram_prec);
+    Schedule sc = build_schedule(rows, ptr, split_len, batch_work, grid, gram_prec, nullptr, batch_work <= 0);
     out->nunits = (int64_t)sc.units.size();
     out->nsplit_rows = (int64_t)sc.splits.size();
     out->nbatches = (int64_t)sc.batch_begin.size() - 1;

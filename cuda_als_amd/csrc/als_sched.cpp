@@ -12,9 +12,8 @@ constexpr int64_t GPU_SIMDS = 1024;  // 256 CUs of four
 int64_t row_solve_cost(int prec) { return prec == PREC_FP32 ? 96 : 1024; }
 
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
-                        const std::vector<int> *subset, bool own_batches, bool slow_ratings) {
+                        const std::vector<int> *subset, bool shrinks, bool slow_ratings) {
     Schedule s;
-    own_batches = own_batches || batch_work <= 0;
     const int64_t solve = row_solve_cost(prec);
     const int64_t nrows = subset ? (int64_t)subset->size() : rows;
     auto row_at = [&](int64_t i) -> int64_t { return subset ? (int64_t)(*subset)[i] : i; };
@@ -60,13 +59,13 @@ Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t
     s.units.reserve(items.size());
     // Batches of batch_work, heaviest rows first. Each batch but a wave's first
     // costs an atomic on a counter that all waves share, some 12 ns, one after
-    // the other. Where the size is the scheduler's own and an average batch is
+    // the other. Where they may shrink (shrinks) and an average batch is
     // little more work than the GPU gets through in that time, the waves would
     // wait for the counter: there the batches start large and shrink to
     // batch_work, each taking half of what an even share of the work still left
     // would be, and small ones are left for the end, to even out what the cost
-    // model got wrong. A caller's size is taken as it is. One half-sweep of
-    // the users, even batches -> shrinking: ml10M shape, f = 64 FP32 838 -> 580
+    // model got wrong. One half-sweep of the
+    // users, even batches -> shrinking: ml10M shape, f = 64 FP32 838 -> 580
     // us (62,600 -> 32,300 batches), f = 16 805 -> 490, f = 80 16-bit Gram and
     // CG 437 -> 289; a quarter of the netflix-shaped users, f = 100 FP32 2.22 ->
     // 2.02 ms. At the whole netflix shape with the 16-bit Gram (items, batches
@@ -105,7 +104,8 @@ Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t
         }
     };
     cut(false);
-    if (own_batches && all < small * (int64_t)s.batch_begin.size()) cut(true);
+    s.shrunk = shrinks && all < small * (int64_t)s.batch_begin.size();
+    if (s.shrunk) cut(true);
     if (s.batch_begin.back() != (int)items.size()) s.batch_begin.push_back((int)items.size());
     return s;
 }

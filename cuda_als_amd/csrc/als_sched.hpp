@@ -10,9 +10,9 @@
 //   * units are ordered by decreasing cost (longest-processing-time first),
 //     so the tail of the launch is made of the lightest rows;
 //   * consecutive units are grouped into batches of `batch_work`
-//     rating-equivalents or just above; where the scheduler chose that size and
-//     it is small, larger batches come first and shrink to it; persistent waves
-//     take batches from a device queue.
+//     rating-equivalents or just above; where they may shrink and that is
+//     small, larger batches come first; persistent waves take batches from a
+//     device queue.
 #pragma once
 #include <cstdint>
 #include <vector>
@@ -39,6 +39,7 @@ struct Schedule {
     int64_t nslots = 0;            // partial-Gram slots needed
     int64_t split_len = 0;
     int64_t batch_work = 0;        // size of a batch; of the smallest where they shrink
+    bool shrunk = false;
 };
 
 // Cost of a solve in rating-equivalents of Gram work for the given Gram
@@ -49,12 +50,11 @@ int64_t row_solve_cost(int prec);
 // split_len <= 0 and batch_work <= 0 select sizes from the total work and
 // the number of persistent waves (`grid`). subset (nullable): schedule only
 // these rows (ascending), e.g. the rows left after the dual system's.
-// own_batches: batch_work is a size that the scheduler chose for an earlier
-// schedule of these rows, and the batches may shrink to it as they may where
-// it is chosen here. slow_ratings: a rating takes well over the model's time
-// (8 or 9 blocks, classic refinement).
+// shrinks: where batches of batch_work would be small, larger ones come first
+// and shrink to it. slow_ratings: a rating takes well over the model's time (8
+// or 9 blocks, classic refinement).
 Schedule build_schedule(int64_t rows, const int *ptr, int64_t split_len, int64_t batch_work, int grid, int prec,
-                        const std::vector<int> *subset = nullptr, bool own_batches = false,
+                        const std::vector<int> *subset = nullptr, bool shrinks = false,
                         bool slow_ratings = false);
 
 }  // namespace als

@@ -210,7 +210,7 @@ int als_schedule_preview(int64_t rows, const int *ptr, int split_len, int batch_
  * Call after als_set_train; results are identical in exact arithmetic for
  * every schedule (split rows sum their parts in a fixed order). */
 typedef struct {
-    int64_t split_len[2], batch_work[2]; /* chosen, per side */
+    int64_t split_len[2], batch_work[2]; /* chosen, per side (as als_set_schedule takes them) */
     float default_ms[2], best_ms[2];     /* one half-sweep: default schedule, chosen one */
     int candidates[2];
     int restage_max[2];                  /* refinement: rows up to this long restage their
@@ -229,10 +229,13 @@ typedef struct {
 int als_autotune(als_engine *e, int sides, als_tune_result *out);
 /* Applies one side's schedule directly (e.g. a stored als_autotune result):
  * split length, batch size (<= 0: keep) and the refinement restage threshold
- * (< 0: keep). Every batch has the size given, but for the one size that the
- * scheduler chose for this side at als_set_train (als_config.batch_work = 0),
- * which brings back the scheduler's own batches: a stored als_autotune result
- * gives the batches that were tuned. No reference counterpart. */
+ * (< 0: keep). Every batch has the size given; with ALS_BATCH_SHRINKS added to
+ * it (by itself: to the size the scheduler chooses) larger ones come first and
+ * shrink to it where it is small, as they do on an engine whose
+ * als_config.batch_work is 0. als_autotune tries sizes in the mode a side is
+ * in and adds the flag where the batches it chose shrink, so that its result
+ * applied here gives them again. No reference counterpart. */
+#define ALS_BATCH_SHRINKS ((int64_t)1 << 40)
 int als_set_schedule(als_engine *e, int side, int64_t split_len, int64_t batch_work, int restage_max);
 /* Update kernel variant of one side: 0 two waves per SIMD for the refinement
  * solvers, 1 one wave per SIMD with the whole register file (warm-started

@@ -1,5 +1,5 @@
 // Prints the batches of one schedule (als_sched.hpp): its batch_work, then
-// batch_begin. Arguments: split_len batch_work grid prec own_batches
+// batch_begin. Arguments: split_len batch_work grid prec shrinks
 // slow_ratings; rating counts of the rows on standard input.
 #include <cstdio>
 #include <cstdlib>

@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 import cuda_als_amd as ca
+from cuda_als_amd import _capi as A
 from cuda_als_amd import engine as E
 from oracle import als_oracle as O
 
@@ -60,19 +61,47 @@ def test_batches_against_waves(f, prec, grid, graph):
             e.set_schedule(ca.ALS_SIDE_USERS, 0, 1)
 
 
+def uneven():
+    rng = np.random.default_rng(9)
+    lengths = rng.integers(1, 200, 3000)
+    idx = np.concatenate([np.sort(rng.choice(500, n, replace=False)) for n in lengths])
+    return ca.from_arrays(3000, 500, np.concatenate([[0], np.cumsum(lengths)]), idx, rng.integers(1, 6, idx.size),
+                          [0], [0], [3.0])
+
+
+def test_batches_shrink_where_they_may():
+    """On 64 waves this matrix's batches, three rows each by the scheduler's
+    choice, shrink from larger ones unless a size is asked for, through the
+    configuration or later; the flag brings the shrinking back, by itself with
+    the scheduler's size, and rebuilds for another grid keep the mode."""
+    d = uneven()
+
+    def batches(cfg, *calls):
+        with E.Engine(E.make_config(16, 0.05, 1, E.SolveType.CHOL, E.Prec.FP32, batch_work=cfg), d) as e:
+            e.set_grid(ca.ALS_SIDE_USERS, 64)
+            for c in calls:
+                e.set_schedule(ca.ALS_SIDE_USERS, 0, c)
+            n = e.info().nbatches[0]
+            e.set_grid(ca.ALS_SIDE_USERS, 63)
+            e.set_grid(ca.ALS_SIDE_USERS, 64)
+            assert e.info().nbatches[0] == n
+            return n
+
+    shrinks = A.ALS_BATCH_SHRINKS
+    assert batches(1) == batches(0, 1) == batches(0, shrinks, 1) == 3000
+    assert batches(1, shrinks + 1) == batches(0, shrinks + 1) < 1500
+    assert batches(1, shrinks) == batches(0, shrinks) < batches(0, 574)
+
+
 @pytest.mark.parametrize("batch_work", [0, 500])
 @pytest.mark.parametrize("prec", [E.Prec.FP32, E.Prec.FP16])
 def test_a_stored_tuning_gives_the_batches_that_were_tuned(prec, batch_work):
     """als_autotune's result applied to a fresh engine in either order of the
-    calls: the same batches as on the tuned engine, also where the scheduler's
-    own (shrinking) ones were the fastest, and the same bits."""
-    rng = np.random.default_rng(9)
-    lengths = rng.integers(1, 200, 3000)
-    idx = np.concatenate([np.sort(rng.choice(500, n, replace=False)) for n in lengths])
-    d = ca.from_arrays(3000, 500, np.concatenate([[0], np.cumsum(lengths)]), idx, rng.integers(1, 6, idx.size),
-                       [0], [0], [3.0])
+    calls: the same batches as on the tuned engine, whether they shrink or
+    not, and the same bits."""
+    d = uneven()
     cfg = E.make_config(70, 0.05, 1, E.SolveType.CHOL, prec, batch_work=batch_work)
-    V0 = rng.standard_normal((500, 70)).astype(np.float32) * 0.3
+    V0 = np.random.default_rng(1).standard_normal((500, 70)).astype(np.float32) * 0.3
 
     def update(e):
         e.set_factors(ca.ALS_SIDE_ITEMS, V0)

@@ -1,6 +1,6 @@
 """The work schedule's batches (no GPU): every rating of every row in exactly
-one unit whatever the batch rule, a caller's batch size kept as it is, the
-scheduler's own batches shrinking where they would be small and even where
+one unit whatever the batch rule, a caller's batch size kept as it is,
+batches that may shrink doing so where they would be small and even where
 they would not, and every unit in exactly one batch."""
 import ctypes as C
 import subprocess
@@ -33,8 +33,8 @@ def batches(tmp_path_factory):
     r = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, r.stderr[-3000:]
 
-    def run(sizes, batch_work, grid, prec, own=False, slow=False):
-        out = subprocess.run([str(exe), "1000000000", str(batch_work), str(grid), str(prec), str(int(own)),
+    def run(sizes, batch_work, grid, prec, shrinks=False, slow=False):
+        out = subprocess.run([str(exe), "1000000000", str(batch_work), str(grid), str(prec), str(int(shrinks)),
                               str(int(slow))],
                              input=" ".join(map(str, sizes)), capture_output=True, text=True, timeout=60, check=True)
         work, *begin = map(int, out.stdout.split())
@@ -79,17 +79,16 @@ def test_small_batches_shrink_from_large_ones(batches):
     size would be one row each. They take half of an even share of what is
     left while that is more than a row: 2 waves' worth of them for every
     factor of e that the work left falls by until it is 2 waves' worth of
-    rows, which go one by one. The same size asked for by a caller is even;
-    kept from an earlier schedule it shrinks again. Rows of 6,000 ratings keep
-    even batches."""
+    rows, which go one by one. The same size asked for without shrinking is
+    even. Rows of 6,000 ratings keep even batches."""
     sizes, waves = np.full(40000, 100), 4096
-    work, begin, cost = batches(sizes, 0, waves, A.ALS_PREC_FP32)
+    work, begin, cost = batches(sizes, 0, waves, A.ALS_PREC_FP32, shrinks=True)
     rows = np.diff(begin)
     assert (np.diff(rows) <= 0).all() and rows[0] > 1 and rows[-1] == 1
     assert rows.size <= 2 * waves * (np.log(40000 / (2 * waves)) + 1) + 1 and work <= cost[0]
     assert (np.diff(batches(sizes, work, waves, A.ALS_PREC_FP32)[1]) == 1).all()
-    assert np.array_equal(batches(sizes, work, waves, A.ALS_PREC_FP32, own=True)[1], begin)
-    _, begin, _ = batches(np.full(4000, 6000), 0, 64, A.ALS_PREC_FP16)
+    assert np.array_equal(batches(sizes, work, waves, A.ALS_PREC_FP32, shrinks=True)[1], begin)
+    _, begin, _ = batches(np.full(4000, 6000), 0, 64, A.ALS_PREC_FP16, shrinks=True)
     assert np.unique(np.diff(begin)[:-1]).size == 1
 
 
@@ -100,7 +99,7 @@ def test_shrinking_batches_are_bounded(prec, most, slow, batches):
     counter asks for (half of that where ratings are slow) by more than its
     last row."""
     sizes = np.random.default_rng(2).poisson(120, 100000)
-    work, begin, cost = batches(sizes, 0, 3072, prec, slow=slow)
+    work, begin, cost = batches(sizes, 0, 3072, prec, True, slow)
     total = np.add.reduceat(cost, begin[:-1])
     bound = most // (1 + slow)
     assert bound <= total.max() < bound + cost.max() and work < bound
