@@ -205,6 +205,7 @@ def adjoint_leg(torch, E, ca, steps, warmup):
         fwd_ms = timed(fwd)
         adj_ms = timed(adj)
         fails = int(e.info().failures)
+    # the saved factors' bytes over the whole adjoint: the solve that reads them and dL/dY's two passes
     out = {"workload": f"ml-latest-shape {d.m}x{d.n}, {d.nnz} train ratings, f={f}, per-user lambda, fp16 Gram, "
                        "fp32 Cholesky; forward = users half-sweep keeping the factors, backward = adjoint",
            "forward_ms": fwd_ms, "adjoint_ms": adj_ms, "saved_factor_bytes": nbytes,
@@ -430,10 +431,10 @@ def main() -> int:
     solve_flops = float(rows) * 2.0 * (f + 1) ** 3 / 3.0
     roof_ms = (gram_flops / (PEAK_FP16_TFLOPS * 1e12) + solve_flops / (PEAK_FP32_TFLOPS * 1e12)) * 1e3
     roofline = {"bound": "mfma", "achieved": achieved, "peak": PEAK_FP16_TFLOPS, "unit": "TFLOP/s",
-                "frac": achieved / PEAK_FP16_TFLOPS, "traffic": parse_traffic(f"update_{half}"),
-                "traffic_source": ("not measured in this run: HBM bytes per launch of the same kernels from "
-                                   "profiles/traffic_update_netflix_shape.md (rocprofv3 --pmc FETCH_SIZE and "
-                                   "WRITE_SIZE, scaled by a plain copy's counters)"),
+                "frac": achieved / PEAK_FP16_TFLOPS, "traffic": parse_traffic(f"update_{half}") if f == 100 else None,
+                "traffic_source": ("not measured in this run: HBM bytes per launch of these kernels (items: the "
+                                   "one-wave kernel) from profiles/traffic_update_netflix_shape.md (rocprofv3 "
+                                   "--pmc FETCH_SIZE and WRITE_SIZE, scaled by a plain copy's counters)"),
                 "kernel": (f"{half} half-sweep: update_kernel (16-bit Gram + Cholesky) and dual_kernel "
                            "(light rows), timed together with HIP events on the engine's stream"),
                 "kernel_ms": ms, "flops_per_launch": gram_flops,
@@ -445,7 +446,7 @@ def main() -> int:
     gather_bytes = float(d.nnz) * (2 * f + 8)
     gbs = gather_bytes / (oms * 1e-3) / 1e12
     roofline_other = {"half": other, "bound": "hbm", "achieved": gbs, "peak": PEAK_HBM_TBS, "unit": "TB/s",
-                      "frac": gbs / PEAK_HBM_TBS, "traffic": parse_traffic(f"update_{other}"),
+                      "frac": gbs / PEAK_HBM_TBS, "traffic": parse_traffic(f"update_{other}") if f == 100 else None,
                       "kernel_ms": oms, "bytes_per_launch": gather_bytes,
                       "note": "the fixed side's 16-bit rows largely come from the Infinity Cache and L2, so "
                               "traffic (L2 misses, from the committed profile) can sit below the algorithmic bytes"}
