@@ -1204,6 +1204,18 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
             }
             return ALS_OK;
         };
+        // After the host's work on a schedule it takes some 20 ms of kernels until
+        // one runs as fast as it does among others. The stages that rebuild none compare like
+        // with like only from there on: with the schedule's first trial among
+        // theirs, the netflix shape's users lost their gathers straight to LDS
+        // (4.41 ms in that trial, 4.12 in sweeps) to those through registers (4.26
+        // and 4.25).
+        auto settle = [&]() -> int {
+            int r = ALS_OK;
+            float t = 0.f;
+            for (float ms = 0.f, k = 0.f; ms < 20.f && k < 200.f && !r; ms += 3.f * t, ++k) r = trial(t);
+            return r;
+        };
         // split length x batch size, under each kernel variant the engine
         // has (the best split length depends on it: a variant's waves take
         // a split row's parts and finishes at their own rate)
@@ -1270,9 +1282,11 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
             const int r0 = s.restage_max;
             int bestr = r0;
             float bestt = 1e30f;
+            rc = settle();
             for (int rm : {r0, 0, 32, 64, 128, 512, 1024, 1 << 30}) {
-                s.restage_max = rm;
                 float t;
+                if (rc) break;
+                s.restage_max = rm;
                 if ((rc = trial(t))) break;
                 if (t < bestt) {
                     bestt = t;
@@ -1290,7 +1304,9 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
             const int v0 = s.variant, d0 = s.gram_dma;
             int bestv = v0, bestd = d0;
             float bestvt = 1e30f;
+            rc = settle();
             for (int v : {v0, 1 - v0}) {
+                if (rc) break;
                 if (v != v0 && e->grid_v1 == 0) continue;
                 for (int dm : {d0, 1 - d0}) {
                     if (dm != d0 && !dma_built) continue;
