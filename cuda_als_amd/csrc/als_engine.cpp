@@ -1356,8 +1356,8 @@ extern "C" int als_autotune(als_engine *e, int sides, als_tune_result *out) {
 // took 29.8 ms per sweep against 26.4 ms for three separate engines (the
 // kernels of then). Inside the capture a model's dual kernel follows its
 // update kernel. At the ml10M shape (BF16, one warm-started step) the group
-// runs 448 sweeps/s of all three models, the engines one after another on one
-// stream 445, on streams of their own, dual kernels beside, 475.
+// runs 447 sweeps/s of all three models, the engines one after another on one
+// stream 446, on streams of their own, dual kernels beside, 475.
 struct als_group {
     std::vector<als_engine *> eng;
     std::vector<hipStream_t> streams;  // one per model
